@@ -188,10 +188,12 @@ _VARIANT_IDS = {"tile128x128_wave64x32": 0, "tile128x128_wave64x64": 0,
 _TILE = {0: (128, 128), 1: (128, 128), 2: (256, 128), 4: (256, 256)}
 _IN_BYTES = {"f32": 4, "f16": 2, "bf16": 2, "fp8": 1}
 _OUT_BYTES = {"f32": 4, "f16": 2, "bf16": 2}
-# own k-tile cycles per (variant, input class 0 16-bit / 1 fp8 / 2 f32),
-# fixed cycles per (variant, epilogue 0 exchange / 1 split), then scalars
-_KT = [(0, 0), (0, 1), (0, 2), (1, 0), (1, 1), (2, 0), (2, 1), (4, 0), (4, 1)]
-_FX = [(0, 0), (0, 1), (1, 0), (1, 1), (2, 1), (4, 1)]
+# own k-tile cycles per (variant, input class 0 16-bit / 1 fp8 / 2 f32 /
+# 3 f32 on 64 x 64 tiles), fixed cycles per (variant, epilogue 0 exchange /
+# 1 split, class 0 16-bit and fp8 / 2, 3 as above), then scalars
+_KT = [(0, 0), (0, 1), (0, 2), (0, 3), (1, 0), (1, 1), (2, 0), (2, 1), (4, 0), (4, 1)]
+_FX = [(0, 0, 0), (0, 1, 0), (0, 0, 2), (0, 1, 2), (0, 0, 3), (1, 0, 0), (1, 1, 0), (2, 1, 0),
+       (4, 1, 0)]
 _SCALARS = ["launch_us", "exchange_us", "exchange_per_tile_us", "hbm_gbs", "feed_gbs",
             "rows_block_cyc", "rows_tile_cyc", "rows_kstep_cyc"]
 
@@ -221,6 +223,10 @@ def model_us(x, r, cu=256):
         return c["launch_us"] + max(waves * cyc / (f * 1e3), (ab + elems * osz) * us_per_byte)
     rows, cols = _TILE[v]
     cls = 1 if r["in"] == "fp8" else (2 if r["in"] == "f32" else 0)
+    if cls == 2 and r["path"] == "exchange" and (
+            b * math.ceil(m / 64) * math.ceil(n / 64) <= 2 * cu and math.ceil(n / 64) <= 64):
+        rows = cols = 64  # tile_shape's rule (csrc/variants.cpp)
+        cls = 3
     n_t = math.ceil(n / cols)
     tiles = b * math.ceil(m / rows) * n_t
     waves = math.ceil(tiles / cu)
@@ -232,9 +238,9 @@ def model_us(x, r, cu=256):
     for count, active in ((full, cu), (1 if rem else 0, rem)):
         if count:
             per_kt = kt[(v, cls)] + (rows + cols) * 128 * active * f / c["feed_gbs"]
-            t_tiles += count * (fx[(v, epi)] + nk * per_kt) / (f * 1e3)
+            t_tiles += count * (fx[(v, epi, cls if cls >= 2 else 0)] + nk * per_kt) / (f * 1e3)
     if r["path"] == "exchange":
-        t_xch = c["exchange_us"] + c["exchange_per_tile_us"] * n_t if n > 128 else 0.0
+        t_xch = c["exchange_us"] + c["exchange_per_tile_us"] * n_t if n > cols else 0.0
         return c["launch_us"] + max(t_tiles, (ab + elems * osz) * us_per_byte) + t_xch
     stats = b * m * n_t * 8
     return (2 * c["launch_us"] + max(t_tiles, (ab + elems * osz + stats) * us_per_byte)
@@ -268,7 +274,8 @@ def _report_fit(files):
     records = [json.loads(line) for f in files for line in open(f) if line.strip()]
     x = fit_constants(records)
     names = ([f"kt_cyc[variant {v}][class {c}]" for v, c in _KT] +
-             [f"fixed_cyc[variant {v}][{'exchange' if e == 0 else 'split'}]" for v, e in _FX] +
+             [f"fixed_cyc[variant {v}][{'exchange' if e == 0 else 'split'}][class {c}]"
+              for v, e, c in _FX] +
              _SCALARS)
     for name, val in zip(names, x):
         print(f"{name:36s} {val:12.4f}")

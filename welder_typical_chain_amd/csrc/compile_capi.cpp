@@ -24,14 +24,14 @@ namespace wtc {
 
 // Workgroup sizes of the kernels (defined with the kernels and the launcher
 // in the library).
-int chain_kernel_threads(int in_dt);
+int chain_kernel_threads(int in_dt, int tile_rows, int loaders);
 int wide_kernel_threads();
 int rows_kernel_threads();
 int rescale_waves_per_row(int64_t rows_total, int cu_count);
 // Compute units of the current device, or `fallback` when no GPU is visible.
 int device_cu_count(int fallback);
-// Dynamic LDS bytes the launcher adds to the exchange kernel of wave layout ks.
-int exchange_lds_pad(int in_dt, int out_dt, int loaders);
+// Dynamic LDS bytes the launcher adds to the exchange kernel of tile ts.
+int exchange_lds_pad(int in_dt, int out_dt, const TileShape& ts, int64_t grid, int cu_count);
 
 static std::string library_path() {
   Dl_info info{};
@@ -115,17 +115,17 @@ struct StageKernel {
 // this build runs them, with this problem's bounds (the reference's file at
 // this stage is its chain lowered to loops; here the loops are those of the
 // hand-written gfx950 kernels, the bodies named by the instructions they issue).
-static std::string emit_loop_structure(const ChainSpec& spec, const VariantDesc& var, int in_code,
+static std::string emit_loop_structure(const ChainSpec& spec, const VariantDesc& var, const TileShape& ts, int in_code,
                                        const char* path, const std::vector<StageKernel>& ks) {
   const int64_t eb = in_code == WTC_DTYPE_FP8_E4M3 ? 1 : in_code == WTC_DTYPE_F32 ? 4 : 2;
   const int64_t tk = 128 / eb;                                  // elements of one 128-byte k-tile
   const int64_t nk = (spec.k * eb + 127) / 128;                 // k-tiles
-  const int64_t tm = var.tile_rows, tn = var.id == kVarTile256x256 ? 256 : 128;
+  const int64_t tm = ts.rows, tn = ts.cols;
   const int64_t rows = spec.batch * spec.m, nT = (spec.n + tn - 1) / tn;
   const char* mfma = in_code == WTC_DTYPE_FP8_E4M3 ? "v_mfma_scale_f32_32x32x64_f8f6f4"
                      : in_code == WTC_DTYPE_BF16 ? "v_mfma_f32_32x32x16_bf16"
-                     : in_code == WTC_DTYPE_F32 ? "v_mfma_f32_32x32x2f32" : "v_mfma_f32_32x32x16_f16";
-  const int64_t ksteps = in_code == WTC_DTYPE_FP8_E4M3 ? 2 : in_code == WTC_DTYPE_F32 ? 16 : 4;
+                     : in_code == WTC_DTYPE_F32 ? "6 x v_mfma_f32_32x32x16_bf16 (three bf16 parts a value)" : "v_mfma_f32_32x32x16_f16";
+  const int64_t ksteps = in_code == WTC_DTYPE_FP8_E4M3 ? 2 : in_code == WTC_DTYPE_F32 ? 2 : 4;
   std::ostringstream o;
   o << "// Loop structure of the " << path << " path's kernels on gfx950 (variant " << var.name
     << "),\n// with this problem's bounds: batch " << spec.batch << ", M " << spec.m << ", N " << spec.n
@@ -153,7 +153,9 @@ static std::string emit_loop_structure(const ChainSpec& spec, const VariantDesc&
       o << "      // workgroup -> (row block, column tile) of " << tm << "x" << tn
         << ", XCD-aware order\n"
         << "      scf.for %kt = %c0 to %nk step %c1 {  // k-tiles of " << tk
-        << " elements: direct-to-LDS buffer loads of k-tile kt+3 into the LDS ring\n"
+        << (in_code == WTC_DTYPE_F32
+                ? " elements: loaded ahead into registers, split into bf16 parts, written to the LDS ring\n"
+                : " elements: direct-to-LDS buffer loads of k-tile kt+3 into the LDS ring\n")
         << "        scf.for %s = %c0 to %ks step %c1 {  // LDS fragment reads (B: ds_read_b64_tr), "
         << mfma << ", f32 accumulators\n        }\n      }\n";
       if (k.kind == "tile_logits") {
@@ -286,10 +288,10 @@ static int compile_impl(const char* input_mlir_path, const char* out_dir, int64_
     int block = 256;
     std::string kind = "rowwise";  // loop structure in 04c (StageKernel::kind)
   };
-  // chain_tile_kernel<in, out, epi, PF = 3, tile rows, ks>
-  auto chain_sym = [](int in, int out, int epi, int tm = 128, int lw = 0) {
+  // chain_tile_kernel<in, out, epi, tile rows, loaders>
+  auto chain_sym = [](int in, int out, int epi, int tm, int lw) {
     return "_ZN3wtc17chain_tile_kernelILi" + std::to_string(in) + "ELi" + std::to_string(out) +
-           "ELi" + std::to_string(epi) + "ELi3ELi" + std::to_string(tm) + "ELi" + std::to_string(lw) + "E";
+           "ELi" + std::to_string(epi) + "ELi" + std::to_string(tm) + "ELi" + std::to_string(lw) + "E";
   };
   // chain_wide_kernel<in, out, epi>: the 256x256 tiles
   auto wide_sym = [](int in, int out, int epi) {
@@ -297,28 +299,30 @@ static int compile_impl(const char* input_mlir_path, const char* out_dir, int64_
            "ELi" + std::to_string(epi) + "E";
   };
   const bool wide = var.id == kVarTile256x256;
+  const TileShape ts = tile_shape(
+      var, path, Problem{spec.batch, spec.m, spec.n, spec.k, in_code, out_code, cu_count, 1});
+  const std::string layout = std::to_string(ts.rows) + "x" + std::to_string(ts.cols) +
+                             (ts.loaders ? (spec.in == Elem::F32 ? ",2 k-groups" : ",loaders") : "");
   // the split / unfused tile kernel of the variant: display name and symbol
   auto tile_kern = [&](int out, const std::string& out_name, int epi, const std::string& epi_name) {
     if (wide) return std::make_pair("chain_wide_kernel<" + kin + "," + out_name + "," + epi_name + ",256x256>",
                                     wide_sym(in_code, out, epi));
-    const std::string layout = std::to_string(var.tile_rows) + "x128" + (var.loaders ? ",loaders" : "");
     return std::make_pair("chain_tile_kernel<" + kin + "," + out_name + "," + epi_name + "," + layout + ">",
-                          chain_sym(in_code, out, epi, var.tile_rows, var.loaders));
+                          chain_sym(in_code, out, epi, ts.rows, ts.loaders));
   };
   const std::string out_t = "ILi" + std::to_string(out_code) + "E";
   std::vector<K> ks;
   const int64_t rows = spec.batch * spec.m;
-  const int tile_threads = wide ? wide_kernel_threads() : chain_kernel_threads(in_code);
+  const int tile_threads = wide ? wide_kernel_threads() : chain_kernel_threads(in_code, ts.rows, ts.loaders);
   if (path == WTC_PATH_ROWS) {
     ks.push_back({"chain_rows_kernel<" + kin + "," + kout + ">",
                   "_ZN3wtc17chain_rows_kernelILi" + std::to_string(in_code) + "ELi" +
                       std::to_string(out_code) + "E",
                   grid, 0, rows_kernel_threads(), "rows"});
   } else if (path == WTC_PATH_EXCHANGE) {
-    ks.push_back({"chain_tile_kernel<" + kin + "," + kout + ",exchange,128x128" +
-                      (var.loaders ? ",loaders" : "") + ">",
-                  chain_sym(in_code, out_code, 0, 128, var.loaders), grid,
-                  exchange_lds_pad(in_code, out_code, var.loaders), tile_threads, "tile_exchange"});
+    const auto tk = tile_kern(out_code, kout, 0, "exchange");
+    ks.push_back({tk.first, tk.second, grid, exchange_lds_pad(in_code, out_code, ts, grid, cu_count),
+                  tile_threads, "tile_exchange"});
   } else if (path == WTC_PATH_SPLIT) {
     const auto tk = tile_kern(out_code, kout, 1, "split");
     ks.push_back({tk.first, tk.second, grid, 0, tile_threads, "tile_split"});
@@ -477,7 +481,7 @@ static int compile_impl(const char* input_mlir_path, const char* out_dir, int64_
         << ")\n";
   }
   run << "    return\n  }\n}\n";
-  const std::string loops = emit_loop_structure(spec, var, in_code, path_name(path), stage_ks);
+  const std::string loops = emit_loop_structure(spec, var, ts, in_code, path_name(path), stage_ks);
   if (!write_file((od / "03.after_postbufferize.mlir").string(), canonical) ||
       !write_file((od / "04.after_workgroup_launch.mlir").string(), wg.str()) ||
       !write_file((od / "04c.after_linalg_to_loops.mlir").string(), loops) ||

@@ -59,6 +59,12 @@ __device__ inline void report_timeout(uint32_t* err, uint32_t* mailbox) {
   if (mailbox) __hip_atomic_fetch_or(mailbox, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// The longest wait, kept in err[1].  One word for the whole grid: same-address
+// atomics take their turns, and when every polling wave sent one (up to 2048)
+// the entries that other waves were still waiting for arrived up to 10 us late
+// behind them (f32 2048 x 1024 x 32 on 512 tiles: 19.0 us a call).  A wave
+// therefore reads the word at the start of the kernel and sends its wait only
+// if it is longer, which after the first calls is rare.
 __device__ inline void record_wait(uint32_t* err, uint64_t ticks) {
   const uint32_t w32 = ticks > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)ticks;
   __hip_atomic_fetch_max(err + 1, w32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -10,11 +10,11 @@
 // path of large problems).  16-bit and fp8 inputs: 512 threads = 8 waves, 2
 // per SIMD (the wave layouts are described at Cfg); k-tiles of 128 bytes of
 // K stream through an LDS ring filled by direct-to-LDS buffer loads, B stays
-// K-major in LDS and its MFMA operands are read with LDS transpose reads.  f32 inputs:
-// 256 threads = 4 waves in a 2x2 grid; k-tiles are loaded `PF` ahead into
-// registers (out-of-range lanes read zero, so the outstanding-load count
-// stays exact), B is transposed in registers, and a two-stage LDS ring feeds
-// the MFMAs.  Accumulation is f32.  The MFMA is issued as D = B^T . A^T so
+// K-major in LDS and its MFMA operands are read with LDS transpose reads.  f32
+// inputs: TM x TM tiles (TM = 64 or 128); k-tiles of 32 are loaded `PF` ahead
+// into registers, each value is split into three bf16 that add up to it
+// exactly, and a two-stage LDS ring of bf16 planes feeds bf16 MFMAs (F32Regs,
+// below).  Accumulation is f32.  The MFMA is issued as D = B^T . A^T so
 // that each lane's accumulators belong to ONE output row: row max / sum are
 // then in-register, one cross-half swap, and one LDS exchange between the
 // waves sharing the row.
@@ -72,10 +72,8 @@ __device__ int64_t g_phase_stamps[kStampTiles * kStampWords];
 #endif
 
 
-constexpr int BM = 128;
-constexpr int BN = 128;
-constexpr int A_STAGE_BYTES = BM * kKTileBytes;                  // 16 KiB
-constexpr int STAGE_BYTES = A_STAGE_BYTES + BN * kKTileBytes;    // 32 KiB
+// Rows of an exchange slot's entries (64-row tiles use the first half).
+constexpr int kSlotRows = 128;
 
 // Per input type, tile height TM and wave layout LW.  16-bit and fp8 inputs
 // stream through a ring of direct-to-LDS loads with 8 waves, 2 per SIMD:
@@ -90,37 +88,47 @@ constexpr int STAGE_BYTES = A_STAGE_BYTES + BN * kKTileBytes;    // 32 KiB
 //     64x32 blocks), and 4 loader waves that issue every direct-to-LDS load,
 //     so an MFMA wave never waits for the memory pipeline to take a load.
 //     All 8 waves share the epilogue's polling, merging and stores.
-// f32 goes through a 2-stage ring filled from registers with 4 waves of
-// 64x64 (TM = 128, LW = 0 only).  Every ring keeps k-tiles kt+1 .. kt+3 in
-// flight or landed while k-tile kt's fragments are in registers, so 3 stages
-// suffice when a stage may be refilled as soon as its fragments have been read.
+// Those rings keep k-tiles kt+1 .. kt+3 in flight or landed while k-tile
+// kt's fragments are in registers, so 3 stages suffice when a stage may be
+// refilled as soon as its fragments have been read.
+// f32 (TM x TM tiles): a 2x2 grid of MFMA waves per k-group.  LW = 0: one
+// group, 4 waves.  LW = 1: two groups, 8 waves; group g runs k-step g of each
+// k-tile's two and the groups' sums meet in LDS after the K loop, so that the
+// value splitting, bound by what one wave can issue, runs on two waves per
+// SIMD.  Group 1 then has no block and takes part in the epilogue as loader
+// waves do.  A stage holds the three bf16 planes of A, [TM rows][64 bytes],
+// and of B, [32 k-rows][2 TM bytes].
 template <int IN_DT, int TM = 128, int LW = 0> struct Cfg {
   static constexpr bool kDma = IN_DT == DT_F16 || IN_DT == DT_BF16 || IN_DT == DT_FP8;
-  static_assert(TM == 128 || (TM == 256 && kDma), "tile height");
-  static_assert(LW == 0 || (LW == 1 && kDma && TM == 128), "loader-wave layout");
-  static constexpr bool kLoaders = LW == 1;
+  static_assert(TM == 128 || (TM == 256 && kDma) || (TM == 64 && !kDma), "tile height");
+  static_assert(LW == 0 || (LW == 1 && TM <= 128), "loader-wave / k-group layout");
+  static constexpr bool kLoaders = LW == 1;  // half of the waves own no block in the epilogue
   static constexpr int kBM = TM;
+  static constexpr int kBN = kDma ? 128 : TM;
   static constexpr int kWavesM = kDma ? TM / 64 : 2;                         // MFMA waves along M
   static constexpr int kWavesN = kLoaders ? 2 : (kDma ? 8 / kWavesM : 2);   // ... along N
   static constexpr int kMfmaWaves = kWavesM * kWavesN;
   static constexpr int kWaves = kLoaders ? 2 * kMfmaWaves : kMfmaWaves;
   static constexpr int kLoadWaves = kLoaders ? kWaves - kMfmaWaves : kWaves;  // issue the loads
   static constexpr int kThreads = 64 * kWaves;
-  static constexpr int kNT = BN / kWavesN / 32;  // 32-column subtiles per MFMA wave
+  static constexpr int kMT = TM / kWavesM / 32;  // 32-row subtiles per MFMA wave
+  static constexpr int kNT = kBN / kWavesN / 32;  // 32-column subtiles per MFMA wave
   // MFMA k-steps of one k-tile (16-bit: 4 of 16; fp8: 2 of 64)
   static constexpr int kKSteps = IN_DT == DT_FP8 ? 2 : 4;
   static constexpr int kABlocksPerWave = TM / 8 / kLoadWaves;  // 1 KiB load blocks of A
   static constexpr int kBBlocksPerWave = 16 / kLoadWaves;      // ... and of B
-  static constexpr int kAStageBytes = TM * kKTileBytes;
-  static constexpr int kStageBytes = kAStageBytes + BN * kKTileBytes;
+  static constexpr int kAPlane = TM * 64, kBPlane = TM * 64;  // f32: bytes of one bf16 plane
+  static constexpr int kAStageBytes = kDma ? TM * kKTileBytes : 3 * kAPlane;
+  static constexpr int kStageBytes = kAStageBytes + (kDma ? kBN * kKTileBytes : 3 * kBPlane);
   static constexpr int kStages = kDma ? (TM == 256 ? 3 : 4) : 2;
   static constexpr int kRingBytes = kStages * kStageBytes;
+  // f32 64 x 64 tiles: registers for two workgroups per CU
+  static constexpr int kWavesPerSimd = TM == 64 ? 2 * kWaves / 4 : 1;
 };
 
 
-// The epilogue stages the tile in LDS as f32 rows of kStagePitch floats (the
+// The epilogue stages the tile in LDS as f32 rows of BN + 4 floats (the
 // 4-float pad spreads the 32 rows one wave writes at a time over all banks).
-constexpr int kStagePitch = BN + 4;
 
 // The exchange path's table of the row block's tile log-sum-exps, [slot][row]
 // with a row pitch of 129 floats (the 4 threads of a row read 4 slots from 4
@@ -128,7 +136,8 @@ constexpr int kStagePitch = BN + 4;
 constexpr int kLsePitch = 129;
 
 template <int IN_DT, int OUT_DT, int TM = 128, int LW = 0, bool XCH = false> struct EpiLayout {
-  static constexpr int STAGING = TM * kStagePitch * 4;
+  static constexpr int PITCH = Cfg<IN_DT, TM, LW>::kBN + 4;  // floats per staged row
+  static constexpr int STAGING = TM * PITCH * 4;
   // exchange path: the log-sum-exp table follows the staged tile
   static constexpr int LSE_OFF = (STAGING + 255) / 256 * 256;
   static constexpr int LSE_END = XCH ? LSE_OFF + 64 * kLsePitch * 4 : STAGING;
@@ -139,74 +148,215 @@ template <int IN_DT, int OUT_DT, int TM = 128, int LW = 0, bool XCH = false> str
   // exchange path's tile log-sum-exps [TM] (float) and slot generations [64]
   static constexpr int TOTAL = RED_OFF + 3 * Cfg<IN_DT, TM, LW>::kWavesN * TM * 4 + TM * 4 + 64 * 4;
   static_assert(TOTAL <= 160 * 1024, "LDS");
-};
-
-// -------------------------------------------------------------------------
-// HBM -> registers -> LDS staging of one k-tile.  Every thread issues the same
-// straight-line sequence: 4 x 128-bit loads of A and one B block (8 x 64-bit
-// for 16-bit types, 16 x 32-bit for fp8, 4 x 128-bit for f32).
-// -------------------------------------------------------------------------
-struct Tile {
-  __amdgpu_buffer_rsrc_t ra, rb;
-  int64_t row0, n0, M, N, K, lda, ldb;
+  // f32 64 x 64 tiles: two workgroups per CU
+  static_assert(TM != 64 || TOTAL <= 80 * 1024, "LDS");
 };
 
 __device__ inline uint32_t bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
 }
 
-template <int IN_DT> struct StageRegs {
-  u32x4 a[4];
-  uint32_t b[16];  // the thread's B k-rows, row-major, 4 columns per row
+// -------------------------------------------------------------------------
+// f32 inputs on the bf16 matrix cores.  A f32 value x is the exact sum of
+// three bf16 values: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1 (8, 8
+// and the last 8 of its 24 significant bits; both differences are exact in
+// f32).  Of the nine partial products of a . b the six of order 2^-18 and
+// above are summed, in f32:
+//   a0 b0 + a0 b1 + a1 b0 + a1 b1 + a0 b2 + a2 b0;
+// what is left out is below 2^-26 |a b|, a quarter of the rounding of one f32
+// product.  Six bf16 MFMAs cost 6/16 of the f32 MFMAs of the same k, and
+// round the accumulator less often (6 times per 16 k, not 8), so the sums are
+// no further from the 64-bit ones than f32 MFMAs leave them (relative 2-norm
+// error of the outputs, N(0, 1) logits, 1024 x 1024 x 1024: 5.5e-7, with f32
+// MFMAs 1.1e-6).
+//
+// Values that do not split: magnitudes below 2^-100 (a part would be subnormal;
+// the least magnitude of the tile's values tells, Tiny) and infinities, NaN and
+// values that round to an infinite x0 (x - x0 is then NaN or infinite, and so
+// is an accumulator at the end).  The workgroup then recomputes its tile with
+// f32 MFMAs (f32_tile_exactly).
+// -------------------------------------------------------------------------
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
-  __device__ inline void load(const Tile& tl, int kt, int t) {
-    constexpr int SZ = dtype_bytes(IN_DT);
-    constexpr int EPC = kChunkBytes / SZ;
-    const int64_t kb = (int64_t)kt * kKTileBytes + a_load_chunk(t) * kChunkBytes;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t row = tl.row0 + a_load_row(t, j);
-      const bool ok = row < tl.M && kb < tl.K * SZ;
-      a[j] = bload16(tl.ra, ok ? (uint32_t)(row * tl.lda + kb) : kOutOfRange);
-    }
-    const int64_t n = tl.n0 + 4 * b_load_colgroup(t);
-    const int64_t k0 = (int64_t)kt * (kKTileBytes / SZ) + b_load_chunkrow(t) * EPC;
-#pragma unroll
-    for (int r = 0; r < EPC; ++r) {
-      const int64_t k = k0 + r;
-      const bool ok = n < tl.N && k < tl.K;
-      const uint32_t off = ok ? (uint32_t)(k * tl.ldb + n * SZ) : kOutOfRange;
-      if constexpr (SZ == 2) {
-        const u32x2 x = bload8(tl.rb, off);
-        b[2 * r] = x[0];
-        b[2 * r + 1] = x[1];
-      } else if constexpr (SZ == 1) {
-        b[r] = bload4(tl.rb, off);
-      } else {
-        const u32x4 x = bload16(tl.rb, off);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) b[4 * r + e] = x[e];
-      }
-    }
+// The least nonzero magnitude seen: as 2 * bits - 1, which puts zero last.
+struct Tiny {
+  uint32_t least = 0xFFFFFFFFu;
+  __device__ inline void see(uint32_t x, uint32_t y) { least = min(least, min((x << 1) - 1u, (y << 1) - 1u)); }
+  __device__ inline bool none() const { return least >= (27u << 24) - 1u; }  // 2^-100
+};
+
+// The three parts of the pair (x, y), each two packed bf16.
+__device__ inline u32x3 split_pair(uint32_t xb, uint32_t yb) {
+  const float x = __builtin_bit_cast(float, xb), y = __builtin_bit_cast(float, yb);
+  const bf16x2 p0 = __builtin_convertvector(f32x2{x, y}, bf16x2);
+  const uint32_t w0 = __builtin_bit_cast(uint32_t, p0);
+  const float x1 = x - __builtin_bit_cast(float, w0 << 16);
+  const float y1 = y - __builtin_bit_cast(float, w0 & 0xFFFF0000u);
+  const bf16x2 p1 = __builtin_convertvector(f32x2{x1, y1}, bf16x2);
+  const uint32_t w1 = __builtin_bit_cast(uint32_t, p1);
+  const float x2 = x1 - __builtin_bit_cast(float, w1 << 16);
+  const float y2 = y1 - __builtin_bit_cast(float, w1 & 0xFFFF0000u);
+  const bf16x2 p2 = __builtin_convertvector(f32x2{x2, y2}, bf16x2);
+  return u32x3{w0, w1, __builtin_bit_cast(uint32_t, p2)};
+}
+
+// Byte offset of column n of k-row k in a plane of B: K-major like the 16-bit
+// tiles' (btr_offset); 64-column tiles keep 128 bytes per k-row and swap its
+// halves by (k / 2) % 2, so that the four k-rows of a transpose read fall in
+// distinct banks.
+template <int TM> __device__ inline int f32_b_offset(int k, int n) {
+  if constexpr (TM == 128) return btr_offset(k, n);
+  return f32_btr64_offset(k, n);
+}
+
+// One k-tile (32 k) of A and B in flight in registers: a thread holds E
+// consecutive k of one row of A and E consecutive columns of one k-row of B.
+// Every load is issued unconditionally (past M, N or K: an offset that reads
+// zero), so the compiler's count of outstanding loads stays exact.
+template <int TM, int NT> struct F32Regs {
+  static constexpr int E = TM * 32 / NT;  // 8 or 4
+  static constexpr int TPA = 32 / E;      // threads per row of A
+  static constexpr int TPB = TM / E;      // threads per k-row of B
+  static constexpr int V = E / 4;
+  u32x4 a[V], b[V];
+
+  struct Where {
+    __amdgpu_buffer_rsrc_t ra, rb;
+    uint32_t a_off, b_off, ldb, K;  // byte offsets of the thread's values in k-tile 0
+    int ak, bk;                     // their first k
+  };
+  static __device__ inline Where where(const void* pa, const void* pb, uint32_t a_bytes, uint32_t b_bytes,
+                                       uint32_t row0, uint32_t n0, uint32_t M, uint32_t N, uint32_t K,
+                                       uint32_t lda, uint32_t ldb, int t) {
+    Where w;
+    w.ra = make_rsrc(pa, a_bytes);
+    w.rb = make_rsrc(pb, b_bytes);
+    w.K = K;
+    w.ldb = ldb;
+    w.ak = (t % TPA) * E;
+    w.bk = t / TPB;
+    const uint32_t row = row0 + (uint32_t)(t / TPA), n = n0 + (uint32_t)((t % TPB) * E);
+    // rows past M start at or past the end of the batch slice: they read zero
+    w.a_off = row < M ? row * lda + (uint32_t)w.ak * 4u : kOutOfRange;
+    w.b_off = n < N ? (uint32_t)w.bk * ldb + n * 4u : kOutOfRange;
+    return w;
   }
-
-  __device__ inline void store(uint8_t* stage, int t) const {
-    constexpr int SZ = dtype_bytes(IN_DT);
+  __device__ inline void load(const Where& w, int kt) {
+    const uint32_t k0 = (uint32_t)kt * 32u;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<u32x4*>(stage + a_lds_offset(a_load_row(t, j), a_load_chunk(t))) = a[j];
-    const int g = b_load_colgroup(t), kc = b_load_chunkrow(t);
-    uint8_t* sB = stage + A_STAGE_BYTES;
-    auto rw = [this](int i) { return b[i]; };
+    for (int i = 0; i < V; ++i) {  // K is a multiple of 4, N of 8
+      const bool ok = w.a_off != kOutOfRange && k0 + (uint32_t)(w.ak + 4 * i) < w.K;
+      a[i] = bload16(w.ra, ok ? w.a_off + k0 * 4u + 16u * i : kOutOfRange);
+    }
+    const bool ok = w.b_off != kOutOfRange && k0 + (uint32_t)w.bk < w.K;
+    const uint32_t off = ok ? w.b_off + k0 * w.ldb : kOutOfRange;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      u32x4 v;
+    for (int i = 0; i < V; ++i) b[i] = bload16(w.rb, off + (ok ? 16u * i : 0u));
+  }
+  // Splits the values and writes their parts to the planes of a stage.
+  __device__ inline void store(uint8_t* stage, int t, Tiny& tiny) const {
+    const int row = t / TPA, ak = (t % TPA) * E, bk = t / TPB, bn = (t % TPB) * E;
+    put(a, stage + a64_lds_offset(row, ak >> 3) + (ak & 7) * 2, Cfg<DT_F32, TM>::kAPlane, tiny);
+    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_offset<TM>(bk, bn), Cfg<DT_F32, TM>::kBPlane, tiny);
+  }
+  static __device__ inline void put(const u32x4 (&v)[V], uint8_t* dst, int plane, Tiny& tiny) {
+    u32x3 w[2 * V];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) v[w] = b_unit_word(rw, SZ, c, w);
-      *reinterpret_cast<u32x4*>(sB + b_lds_offset(kc, 4 * g + c, BN)) = v;
+    for (int i = 0; i < V; ++i) {
+      const u32x4 x = v[i];
+      tiny.see(x[0], x[1]);
+      w[2 * i] = split_pair(x[0], x[1]);
+      tiny.see(x[2], x[3]);
+      w[2 * i + 1] = split_pair(x[2], x[3]);
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      if constexpr (V == 2)
+        *reinterpret_cast<u32x4*>(dst + p * plane) = u32x4{w[0][p], w[1][p], w[2][p], w[3][p]};
+      else
+        *reinterpret_cast<u32x2*>(dst + p * plane) = u32x2{w[0][p], w[1][p]};
     }
   }
 };
+
+__device__ inline f32x16 mfma_bf16(const u32x4& b, const u32x4& a, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c,
+                                                 0, 0, 0);
+}
+
+// A wave's fragments of the k-steps s0 .. s0 + KS - 1 of a stage, per plane.
+template <int TM, int MT, int NTN, int KS> struct F32Frags {
+  u32x4 a[KS][3][MT], b[KS][3][NTN];
+  __device__ inline void read(const uint8_t* stage, int lane, int wm, int nw, int s0) {
+    constexpr int AP = Cfg<DT_F32, TM>::kAPlane, BP = Cfg<DT_F32, TM>::kBPlane;
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const int s = s0 + i;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          a[i][p][mt] = *reinterpret_cast<const u32x4*>(
+              stage + p * AP + a64_lds_offset(wm * 32 * MT + mt * 32 + frag_row(lane), frag64_chunk16(lane, s)));
+#pragma unroll
+        for (int nt = 0; nt < NTN; ++nt) {
+          const uint8_t* sb = stage + 3 * AP + p * BP;
+          const u32x2 lo = tr_read(sb + f32_b_offset<TM>(btr_k(s, 0, lane), btr_n(nw + nt * 32, lane)));
+          const u32x2 hi = tr_read(sb + f32_b_offset<TM>(btr_k(s, 1, lane), btr_n(nw + nt * 32, lane)));
+          b[i][p][nt] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+      }
+  }
+  // The six partial products of every subtile, smallest first.
+  __device__ inline void products(f32x16 (&acc)[MT][NTN]) const {
+    constexpr int kA[6] = {2, 0, 1, 1, 0, 0}, kB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int u = 0; u < 6; ++u)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < NTN; ++nt)
+            acc[mt][nt] = mfma_bf16(b[i][kB[u]][nt], a[i][kA[u]][mt], acc[mt][nt]);
+  }
+};
+
+// The wave's block with f32 MFMAs, operands straight from memory: for tiles
+// with values that do not split.  k-group g of `groups` takes every
+// `groups`-th pair of k.
+template <int MT, int NTN>
+__device__ inline void f32_tile_exactly(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, uint32_t row,
+                                        uint32_t col, uint32_t M, uint32_t N, uint32_t K, uint32_t lda,
+                                        uint32_t ldb, int lane, int g, int groups, f32x16 (&acc)[MT][NTN]) {
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.0f;
+  for (uint32_t kp = 2u * (uint32_t)g; kp < K; kp += 2u * (uint32_t)groups) {
+    const uint32_t k = kp + (uint32_t)(lane >> 5);
+    float a[MT], b[NTN];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const uint32_t r = row + (uint32_t)(mt * 32 + (lane & 31));
+      const uint32_t x = bload4(ra, r < M && k < K ? r * lda + k * 4u : kOutOfRange);
+      a[mt] = __builtin_bit_cast(float, x);
+    }
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt) {
+      const uint32_t n = col + (uint32_t)(nt * 32 + (lane & 31));
+      const uint32_t x = bload4(rb, n < N && k < K ? k * ldb + n * 4u : kOutOfRange);
+      b[nt] = __builtin_bit_cast(float, x);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NTN; ++nt)
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[nt], a[mt], acc[mt][nt], 0, 0, 0);
+  }
+}
 
 // -------------------------------------------------------------------------
 // Direct-to-LDS staging (16-bit inputs).  The loads are issued from inline
@@ -312,110 +462,6 @@ struct DmaPlan {
     for (int j = 0; j < LPT; ++j) issue_one(stage, kt, j);
   }
 };
-
-struct Frags;
-__device__ inline void read_frags_tr(const uint8_t* stage, int lane, int wm, int wn, int s, Frags& f);
-
-// -------------------------------------------------------------------------
-// MFMA over one LDS stage: wave (wm, wn) accumulates its 64x64 block.
-// acc[mt][nt] holds D = B^T A^T for m-subtile mt, n-subtile nt.
-// Fragments of step s+1 are read while the MFMAs of step s issue.
-// -------------------------------------------------------------------------
-struct Frags {
-  u32x4 a[2], b[2];
-};
-
-__device__ inline void read_frags(const uint8_t* stage, int lane, int wm, int wn, int s, Frags& f) {
-  const uint8_t* sA = stage;
-  const uint8_t* sB = stage + A_STAGE_BYTES;
-  const int r = frag_row(lane);
-  const int kch = frag_chunk(lane, s);
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-    f.a[mt] = *reinterpret_cast<const u32x4*>(sA + a_lds_offset(wm * 64 + mt * 32 + r, kch));
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt)
-    f.b[nt] = *reinterpret_cast<const u32x4*>(sB + b_lds_offset(kch, wn * 64 + nt * 32 + r, BN));
-}
-
-// 16-bit fragments with B read K-major through the transpose read.
-__device__ inline void read_frags_tr(const uint8_t* stage, int lane, int wm, int wn, int s, Frags& f) {
-  const uint8_t* sA = stage;
-  const uint8_t* sB = stage + A_STAGE_BYTES;
-  const int r = frag_row(lane);
-  const int kch = frag_chunk(lane, s);
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-    f.a[mt] = *reinterpret_cast<const u32x4*>(sA + a_lds_offset(wm * 64 + mt * 32 + r, kch));
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
-    const int nb = wn * 64 + nt * 32;
-    const u32x2 lo = tr_read(sB + btr_offset(btr_k(s, 0, lane), btr_n(nb, lane)));
-    const u32x2 hi = tr_read(sB + btr_offset(btr_k(s, 1, lane), btr_n(nb, lane)));
-    f.b[nt] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-  }
-}
-
-template <int IN_DT>
-__device__ inline void mma_step(const Frags& f, f32x16 (&acc)[2][2]) {
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      if constexpr (IN_DT == DT_F16) {
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            __builtin_bit_cast(f16x8, f.b[nt]), __builtin_bit_cast(f16x8, f.a[mt]), acc[mt][nt], 0, 0, 0);
-      } else if constexpr (IN_DT == DT_BF16) {
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            __builtin_bit_cast(bf16x8, f.b[nt]), __builtin_bit_cast(bf16x8, f.a[mt]), acc[mt][nt], 0, 0, 0);
-      } else {
-        const u32x4 bv = f.b[nt], av = f.a[mt];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t bw = bv[e], aw = av[e];
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-              __builtin_bit_cast(float, bw), __builtin_bit_cast(float, aw), acc[mt][nt], 0, 0, 0);
-        }
-      }
-    }
-}
-
-__device__ inline void mma_step_fp8(const Frags& f0, const Frags& f1, f32x16 (&acc)[2][2]) {
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const u32x4 a0 = f0.a[mt], a1 = f1.a[mt], b0 = f0.b[nt], b1 = f1.b[nt];
-      const i32x8 av = {(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3],
-                        (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
-      const i32x8 bv = {(int)b0[0], (int)b0[1], (int)b0[2], (int)b0[3],
-                        (int)b1[0], (int)b1[1], (int)b1[2], (int)b1[3]};
-      acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bv, av, acc[mt][nt], 0, 0, 0, 0, 0, 0);
-    }
-}
-
-template <int IN_DT>
-__device__ inline void mma_stage(const uint8_t* stage, int lane, int wm, int wn,
-                                 f32x16 (&acc)[2][2]) {
-  constexpr int S = kChunksPerKTile / 2;  // chunk-pair steps per k-tile
-  Frags f[2];
-  read_frags(stage, lane, wm, wn, 0, f[0]);
-  if constexpr (IN_DT == DT_FP8) {
-#pragma unroll
-    for (int s = 0; s < S; s += 2) {
-      read_frags(stage, lane, wm, wn, s + 1, f[1]);
-      const Frags cur = f[0];
-      if (s + 2 < S) read_frags(stage, lane, wm, wn, s + 2, f[0]);
-      mma_step_fp8(cur, f[1], acc);
-    }
-  } else {
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      if (s + 1 < S) read_frags(stage, lane, wm, wn, s + 1, f[(s + 1) & 1]);
-      mma_step<IN_DT>(f[s & 1], acc);
-    }
-  }
-}
 
 // All MFMA operands of one k-tile for one wave: A fragments [step][m-subtile],
 // B fragments [step][n-subtile], for the wave's KSW k-steps.
@@ -549,18 +595,21 @@ constexpr int step_groups(int loads, int reads, int mfmas) {
 // workgroup count (gridDim.x would be read from the hidden kernel arguments
 // in memory).  Sizes and per-batch strides are 32-bit: the launcher keeps one
 // batch slice of A, B and out below 2 GiB.
-template <int IN_DT, int OUT_DT, int EPI, int PF, int TM, int LW>
-__global__ void __launch_bounds__((Cfg<IN_DT, TM, LW>::kThreads), 1)
+template <int IN_DT, int OUT_DT, int EPI, int TM, int LW>
+__global__ void __launch_bounds__((Cfg<IN_DT, TM, LW>::kThreads), (Cfg<IN_DT, TM, LW>::kWavesPerSimd))
 chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32_t N32,
                   uint32_t K32, uint32_t lda32, uint32_t ldb32, uint32_t nT32, uint32_t nRB32,
                   uint32_t a_bs32, uint32_t b_bs32, uint32_t grid32, const ChainParams p) {
   using C = Cfg<IN_DT, TM, LW>;
   using L = EpiLayout<IN_DT, OUT_DT, TM, LW, EPI == kEpiExchange>;
-  static_assert(EPI != kEpiExchange || TM == 128, "the exchange path runs 128-row tiles");
-  constexpr int BM = TM;  // tile rows
+  static_assert(EPI != kEpiExchange || TM <= kSlotRows, "rows of an exchange slot");
+  constexpr int BM = TM;      // tile rows
+  constexpr int BN = C::kBN;  // tile columns
   constexpr int NT = C::kThreads;
   constexpr int WN = C::kWavesN;  // MFMA waves along N
+  constexpr int MT = C::kMT;      // 32-row subtiles per MFMA wave
   constexpr int NTN = C::kNT;     // 32-column subtiles per MFMA wave
+  constexpr int WM = 32 * MT;     // rows of an MFMA wave's block
   constexpr bool LDW = C::kLoaders;
   __shared__ __attribute__((aligned(16))) uint8_t smem[L::TOTAL];
   float2* wstat = reinterpret_cast<float2*>(smem + L::RED_OFF);  // [WN][BM] wave (max, sum)
@@ -569,10 +618,11 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = t >> 6;
-  // MFMA wave = wm * WN + wn owns rows wm*64 .. +63 and columns nw .. nw +
+  // MFMA wave = wm * WN + wn owns rows wm*WM .. +WM-1 and columns nw .. nw +
   // 32*NTN - 1 of the tile; with loader waves (LW = 1) waves kMfmaWaves ..
-  // issue the loads and own no block (their wm, wn are not used).
-  const int wm = wave / WN, wn = wave % WN;
+  // issue the loads and own no block (their wm, wn are not used), and for
+  // f32 they are the second k-group of the block of wave - kMfmaWaves.
+  const int wm = (C::kDma ? wave : wave % C::kMfmaWaves) / WN, wn = wave % WN;
   const int nw = wn * 32 * NTN;  // first column of the wave's block
   const bool loader = LDW && __builtin_amdgcn_readfirstlane(wave) >= C::kMfmaWaves;
 
@@ -600,15 +650,18 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   // load's destination register -- the compiler waits for it right there.
   const uint32_t slot0 = rbg * nT32;
   uint32_t gen_lane = 0;
+  uint32_t wait_known = 0;  // the longest wait recorded before this launch (record_wait)
   auto load_gen0 = [&]() {
-    if constexpr (EPI == kEpiExchange)
+    if constexpr (EPI == kEpiExchange) {
+      wait_known = __hip_atomic_load(p.err + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       gen_lane = __hip_atomic_load(p.gen + slot0 + ((uint32_t)lane < nT32 ? (uint32_t)lane : nT32 - 1),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   };
 
-  f32x16 acc[2][NTN];
+  f32x16 acc[MT][NTN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NTN; ++j)
 #pragma unroll
@@ -725,53 +778,116 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
     load_gen0();
   } else {
     load_gen0();
-    // ---- main loop, fp8 / f32: PF k-tiles in registers, 2-stage LDS ring --
-    // k-tile j lives in R[j % PF] and is loaded PF-1 iterations before the
-    // iteration that moves it to LDS.  Loads past the last k-tile read zeros
-    // (buffer range check), so the steady-state loop issues every load and
-    // store unconditionally and the compiler's count of outstanding loads
-    // stays exact; the last nk % PF k-tiles run in a guarded tail.
-    static_assert(NT == 256 && NTN == 2, "register path layout");
-    Tile tl;
-    tl.ra = make_rsrc(a_in + (uint64_t)bt * a_bs32, a_bs32);
-    tl.rb = make_rsrc(b_in + (uint64_t)bt * b_bs32, b_bs32);
-    tl.row0 = row0;
-    tl.n0 = n0;
-    tl.M = M32;
-    tl.N = N32;
-    tl.K = K32;
-    tl.lda = lda32;
-    tl.ldb = ldb32;
-    StageRegs<IN_DT> R[PF];
+    // ---- main loop, f32: k-tiles through registers and a ring of bf16 planes ---
+    // k-tile j is requested into R[j % PF], PF iterations before the iteration
+    // that splits it into stage j % 2.  Iteration kt runs k-tile kt's MFMAs and
+    // splits k-tile kt+1 meanwhile.  Loads past the last k-tile read zeros into
+    // a stage that no MFMA uses, so every iteration is the same straight-line
+    // code.
+    // Measured against f32 MFMAs on 128 x 128 tiles (us a call): 1024 x 1024 x
+    // 1024 80.6 -> 22.8 (256 tiles of 64 instead of 64 of 128), 2048 x 2048 x
+    // 1024 82 -> 54, 4096 x 4096 x 512 193 -> 140, 128 x 128 x 128 14.7 -> 8.1.
+    // A 64 x 64 tile's iteration (0.4 us) is bound by LDS: 48 KiB of fragment
+    // reads and 24 KiB of writes, about 650 cycles at the rate LDS delivers,
+    // against 384 cycles of MFMAs; fragments read an iteration ahead (a third
+    // stage) took longer, 23.5 us.  A 128 x 128 tile's (1.3 us) is bound by its
+    // 48 MFMAs a wave, 1536 cycles at the 1.5-1.6 GHz the chip then holds.
+    constexpr int PF = TM == 64 ? 4 : 3;  // k-tiles in registers
+    constexpr int GROUPS = LDW ? 2 : 1;   // k-groups
+    constexpr int STAGE = C::kStageBytes;
+    using Regs = F32Regs<TM, NT>;
+    using Frags = F32Frags<TM, MT, NTN, 2 / GROUPS>;
+    const int kg = loader ? 1 : 0;
+    const uint8_t* a_b = a_in + (uint64_t)bt * a_bs32;
+    const uint8_t* b_b = b_in + (uint64_t)bt * b_bs32;
+    const typename Regs::Where w =
+        Regs::where(a_b, b_b, a_bs32, b_bs32, (uint32_t)row0, (uint32_t)n0, M32, N32, K32, lda32, ldb32, t);
+    uint32_t* redo = reinterpret_cast<uint32_t*>(smem + L::RED_OFF);  // a value of the tile does not split
+    if (t == 0) *redo = 0u;
+    Tiny tiny;
+    Regs R[PF];
 #pragma unroll
-    for (int q = 0; q < PF; ++q) R[q].load(tl, q, t);
-    R[0].store(smem, t);
-    R[0].load(tl, PF, t);
-    __syncthreads();
-    const int nfull = nk - nk % PF;
-    for (int t0 = 0; t0 < nfull; t0 += PF) {
+    for (int q = 0; q < PF; ++q) R[q].load(w, q);
+    auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    R[0].store(smem, t, tiny);
+    R[0].load(w, PF);
+    meet();
+    auto iteration = [&](auto q_c, int kt) {
+      constexpr int Q = decltype(q_c)::value;  // kt % PF
+      Frags F;
+      F.read(smem + (kt & 1) * STAGE, lane, wm, nw, kg);
+      F.products(acc);
+      R[(Q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE, t, tiny);
+      R[(Q + 1) % PF].load(w, kt + 1 + PF);
+      // The scheduler's order: the fragment reads, then the splitting spread
+      // over the MFMAs.  In source order a wave would first issue its MFMAs,
+      // each waiting for the one before it, and only then the arithmetic.
+      constexpr int MF = 6 * MT * NTN * (2 / GROUPS);  // MFMAs
+      constexpr int VA = 4 * Regs::V * 14 + 20;        // VALU instructions, about
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * (MT + 2 * NTN) * (2 / GROUPS), 0);  // LDS reads
 #pragma unroll
-      for (int q = 0; q < PF; ++q) {
-        const int kt = t0 + q;
-        mma_stage<IN_DT>(smem + (kt & 1) * STAGE_BYTES, lane, wm, wn, acc);
-        R[(q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE_BYTES, t);
-        R[(q + 1) % PF].load(tl, kt + 1 + PF, t);
-        __syncthreads();
+      for (int i = 0; i < MF; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, (VA + MF - 1) / MF, 0);  // VALU
+      }
+      meet();
+    };
+    for (int kt = 0;;) {
+      iteration(std::integral_constant<int, 0>{}, kt);
+      if (++kt == nk) break;
+      iteration(std::integral_constant<int, 1>{}, kt);
+      if (++kt == nk) break;
+      iteration(std::integral_constant<int, 2>{}, kt);
+      if (++kt == nk) break;
+      if constexpr (PF == 4) {
+        iteration(std::integral_constant<int, 3>{}, kt);
+        if (++kt == nk) break;
       }
     }
+    bool fine = tiny.none();
 #pragma unroll
-    for (int q = 0; q + 1 < PF; ++q) {
-      const int kt = nfull + q;
-      if (kt < nk) {
-        mma_stage<IN_DT>(smem + (kt & 1) * STAGE_BYTES, lane, wm, wn, acc);
-        R[(q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE_BYTES, t);
-        __syncthreads();
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int j = 0; j < NTN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) fine &= __builtin_isfinite(acc[mt][j][v]);
+    if (!fine) *redo = 1u;
+    meet();
+    if (*redo)
+      f32_tile_exactly<MT, NTN>(w.ra, w.rb, (uint32_t)row0 + (uint32_t)(wm * WM), (uint32_t)(n0 + nw), M32, N32,
+                                K32, lda32, ldb32, lane, kg, GROUPS, acc);
+    if constexpr (GROUPS == 2) {
+      // the groups' sums meet through the ring, 16 bytes per lane per step
+      f32x4* mrg = reinterpret_cast<f32x4*>(smem) + (wave % C::kMfmaWaves) * (MT * NTN * 4 * 64) + lane;
+      if (loader) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < NTN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+              mrg[((mt * NTN + j) * 4 + g) * 64] = f32x4{acc[mt][j][4 * g], acc[mt][j][4 * g + 1],
+                                                        acc[mt][j][4 * g + 2], acc[mt][j][4 * g + 3]};
+      }
+      meet();
+      if (!loader) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < NTN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const f32x4 x = mrg[((mt * NTN + j) * 4 + g) * 64];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[mt][j][4 * g + e] += x[e];
+            }
       }
     }
+    meet();  // the ring and the flag are free
   }
 
   // ---- epilogue --------------------------------------------------------------
-  // Lane owns output rows m_loc(mt) = wm*64 + mt*32 + lane%32 and, for each
+  // Lane owns output rows m_loc(mt) = wm*WM + mt*32 + lane%32 and, for each
   // n-subtile j, the 16 columns n_loc = nw + j*32 + acc_i(lane, v).  Each
   // wave normalises its exponentials against the max of its own columns
   // (wave max m_w, sum s_w per row, kept in LDS); the tile's statistics and
@@ -788,7 +904,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   const int nvalid = p.N - n0 < BN ? (int)(p.N - n0) : BN;  // columns of this tile inside N
   if constexpr (EPI == kEpiLogits) {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int j = 0; j < NTN; ++j)
 #pragma unroll
@@ -804,7 +920,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       const float pad = c2 < 0.0f ? INFINITY : -INFINITY;
       const bool zero = p.c2 == 0.0f;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int j = 0; j < NTN; ++j)
 #pragma unroll
@@ -824,9 +940,9 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       // partial extremes per subtile (one on the 256-row layout, whose
       // waves have no registers to spare)
       constexpr int PX = TM == 256 ? 1 : 4;
-      float ext[2];
+      float ext[MT];
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
+      for (int mt = 0; mt < MT; ++mt) {
         // the row's extreme accumulator over the wave's columns (lane l and
         // l ^ 32 hold the two halves of the row)
         float ex[PX];
@@ -842,9 +958,9 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         for (int i = 1; i < PX; ++i) ext[mt] = pick(ext[mt], ex[i]);
       }
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) ext[mt] = NEG ? xor32_min(ext[mt]) : xor32_max(ext[mt]);
+      for (int mt = 0; mt < MT; ++mt) ext[mt] = NEG ? xor32_min(ext[mt]) : xor32_max(ext[mt]);
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
+      for (int mt = 0; mt < MT; ++mt) {
         // max of y; -inf when every column of the wave lies past N (pad * c2)
         const float mx = ext[mt] * c2;
         const float nbase = mx == -INFINITY ? 0.0f : -mx;
@@ -858,7 +974,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
             s4[v & 3] += e;
           }
         const float sm = xor32_sum((s4[0] + s4[1]) + (s4[2] + s4[3]));
-        if (lane < 32) wstat[wn * BM + wm * 64 + mt * 32 + jr] = make_float2(mx, sm);
+        if (lane < 32) wstat[wn * BM + wm * WM + mt * 32 + jr] = make_float2(mx, sm);
       }
     };
     if (!loader) {
@@ -904,7 +1020,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         // publish the row's log-sum-exp over this tile with this launch's tag
         const float lse = st.x + __builtin_amdgcn_logf(st.y);
         lse_all[nt * kLsePitch + t] = lse;
-        if (!solo) store_entry(p.ent + (uint64_t)own_slot * BM + t, lse, sgen[nt] + 1u);
+        if (!solo) store_entry(p.ent + (uint64_t)own_slot * kSlotRows + t, lse, sgen[nt] + 1u);
         // Wait until the entry stores are acknowledged.  Not for ordering --
         // the tags make every entry self-describing -- but measured: without
         // the wait, entries became visible to the other XCDs late on some
@@ -923,14 +1039,14 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   float* stg = reinterpret_cast<float*>(smem);
   auto stage_tile = [&]() {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int j = 0; j < NTN; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const int m_loc = wm * 64 + mt * 32 + jr;
+          const int m_loc = wm * WM + mt * 32 + jr;
           const int n_loc = nw + j * 32 + acc_i(lane, 4 * g);
-          *reinterpret_cast<f32x4*>(stg + m_loc * kStagePitch + n_loc) =
+          *reinterpret_cast<f32x4*>(stg + m_loc * L::PITCH + n_loc) =
               f32x4{acc[mt][j][4 * g], acc[mt][j][4 * g + 1], acc[mt][j][4 * g + 2],
                     acc[mt][j][4 * g + 3]};
         }
@@ -938,22 +1054,24 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
 
   // Exchange path: poll the other tiles' half-slots of the row block into
   // the table.  Polling wave pw of NWP takes half-slots hs = pw, pw + NWP,
-  // ... (slot hs / 2, rows (hs % 2) * 64 + lane), U at a time: one wave load
+  // ... (slot hs >> HSH, rows 64 (hs mod HS) + lane), U at a time: one wave load
   // is 64 consecutive rows of one slot (512 contiguous bytes), and a
   // half-slot is done when every lane's entry carries the expected tag;
   // otherwise the wave sleeps briefly and reloads only what is not done.
   auto poll_table = [&](int pw_any, int NWP) {
     constexpr int U = 8;
+    constexpr int HS = BM / 64;          // half-slots in use per slot
+    constexpr int HSH = BM == 64 ? 0 : 1;  // its logarithm
     const int pw = __builtin_amdgcn_readfirstlane(pw_any);  // wave-uniform: scalar branches
     const int nT = (int)nT32;
     bool in_time = true;
     uint64_t waited = 0;
-    for (int hb = pw; hb < 2 * nT; hb += U * NWP) {
+    for (int hb = pw; hb < HS * nT; hb += U * NWP) {
       bool done[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int hs = hb + NWP * u;
-        done[u] = !(hs < 2 * nT && (hs >> 1) != (int)nt);  // wave-uniform
+        done[u] = !(hs < HS * nT && (hs >> HSH) != (int)nt);  // wave-uniform
       }
       const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
       for (;;) {
@@ -962,16 +1080,16 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         for (int u = 0; u < U; ++u) {
           const int hs = hb + NWP * u;
           if (!done[u])
-            e[u] = load_entry(p.ent + (uint64_t)(slot0 + (hs >> 1)) * BM + (hs & 1) * 64 + lane);
+            e[u] = load_entry(p.ent + (uint64_t)(slot0 + (hs >> HSH)) * kSlotRows + (hs & (HS - 1)) * 64 + lane);
         }
         bool all = true;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int hs = hb + NWP * u, q = hs >> 1;
+          const int hs = hb + NWP * u, q = hs >> HSH;
           if (!done[u]) {
             if (__all(entry_tag(e[u]) == sgen[q] + 1u) || !in_time) {
               done[u] = true;
-              lse_all[q * kLsePitch + (hs & 1) * 64 + lane] = entry_lse(e[u]);
+              lse_all[q * kLsePitch + (hs & (HS - 1)) * 64 + lane] = entry_lse(e[u]);
             } else {
               all = false;
             }
@@ -984,10 +1102,8 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         if (w > p.spin_ticks) in_time = false;  // one more pass takes what is there
       }
     }
-    if (lane == 0 && waited > 0) {
-      record_wait(p.err, waited);
-      if (!in_time) report_timeout(p.err, p.mailbox);
-    }
+    if (lane == 0 && waited > wait_known) record_wait(p.err, waited);
+    if (lane == 0 && !in_time) report_timeout(p.err, p.mailbox);
   };
 
   if constexpr (EPI == kEpiExchange && LDW) {
@@ -1022,10 +1138,13 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   }
 
   if constexpr (EPI != kEpiLogits) {
-    constexpr int P = NT / BM;  // threads per row (WN, or 2 WN with loader waves)
-    static_assert(P % WN == 0 && (P & (P - 1)) == 0 && P <= 4, "threads per row");
+    // threads per row (WN, or 2 WN with loader waves; at most a quad)
+    constexpr int P = NT / BM < 4 ? NT / BM : 4;
+    static_assert(P % WN == 0 && (P & (P - 1)) == 0 && P * BM % 64 == 0, "threads per row");
     const int r = t / P, h = t % P;
-    if constexpr (EPI == kEpiExchange) {
+    if (P * BM < NT && t >= P * BM) {
+      // 64-row tiles: whole waves without a row
+    } else if constexpr (EPI == kEpiExchange) {
       float gm = -INFINITY, gs = 0.0f;  // running max and sum of exp2(L - gm)
       if (solo) {
         if (h == 0) {  // the row's statistics from this tile's wave entries in LDS
@@ -1069,11 +1188,12 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
 #pragma unroll
       for (int off = 1; off < P; off <<= 1) S += off == 1 ? dpp_quad<0xB1>(S) : dpp_quad<0x4E>(S);
       // thread (r, h < WN) owns the factor of row r, column slice of wave h:
-      // exp2(m_w - L) with L = max + log2(sum) the row's log-sum-exp
-      const float row_lse = M + __builtin_amdgcn_logf(S);
+      // exp2(m_w - M) / S.  (Not exp2(m_w - (M + log2 S)): rounding that sum to
+      // f32 costs up to 3e-7 of the output once the row is a few hundred wide.)
+      const float inv = __builtin_amdgcn_rcpf(S);
       if (h < WN) {
         const float mw = wstat[h * BM + r].x;
-        factor[h * BM + r] = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw - row_lse);
+        factor[h * BM + r] = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw - M) * inv;
       }
     } else {
       // split: exponentials relative to the tile max, as the statistics say
@@ -1120,7 +1240,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       const float f = EPI == kEpiLogits ? 1.0f
                       : factor[(ch * EPC / (32 * NTN)) * BM + row] *
                             (EPI == kEpiSplit ? split_store_scale(OUT_DT) : 1.0f);
-      const float* src = stg + row * kStagePitch + ch * EPC;
+      const float* src = stg + row * L::PITCH + ch * EPC;
       if constexpr (OSZ == 4) {
         const f32x4 x0 = *reinterpret_cast<const f32x4*>(src) * f;
         store16(o_base + m * p.ldo_bytes + n * OSZ, __builtin_bit_cast(u32x4, x0));
@@ -1255,11 +1375,9 @@ __global__ void zero_words_kernel(uint32_t* __restrict__ p, int64_t n) {
 // -------------------------------------------------------------------------
 // Instantiation table
 // -------------------------------------------------------------------------
-constexpr int kPF = 3;
-
 template <int IN_DT, int OUT_DT, int EPI, int TM, int LW>
 static const void* tile_kernel_ptr() {
-  return reinterpret_cast<const void*>(&chain_tile_kernel<IN_DT, OUT_DT, EPI, kPF, TM, LW>);
+  return reinterpret_cast<const void*>(&chain_tile_kernel<IN_DT, OUT_DT, EPI, TM, LW>);
 }
 
 template <int IN_DT, int EPI, int TM, int LW>
@@ -1275,7 +1393,6 @@ static const void* by_out(int out_dt) {
 template <int EPI>
 static const void* by_in(int in_dt, int out_dt) {
   switch (in_dt) {
-    case DT_F32: return by_out<DT_F32, EPI, 128, 0>(out_dt);
     case DT_F16: return by_out<DT_F16, EPI, 128, 0>(out_dt);
     case DT_BF16: return by_out<DT_BF16, EPI, 128, 0>(out_dt);
     case DT_FP8: return by_out<DT_FP8, EPI, 128, 0>(out_dt);
@@ -1283,10 +1400,11 @@ static const void* by_in(int in_dt, int out_dt) {
   return nullptr;
 }
 
-// 128-row tiles with loader waves (16-bit and fp8 inputs).
+// 128-row tiles with loader waves (16-bit and fp8 inputs) or two k-groups (f32).
 template <int EPI>
 static const void* loaders_by_in(int in_dt, int out_dt) {
   switch (in_dt) {
+    case DT_F32: return by_out<DT_F32, EPI, 128, 1>(out_dt);
     case DT_F16: return by_out<DT_F16, EPI, 128, 1>(out_dt);
     case DT_BF16: return by_out<DT_BF16, EPI, 128, 1>(out_dt);
     case DT_FP8: return by_out<DT_FP8, EPI, 128, 1>(out_dt);
@@ -1309,6 +1427,9 @@ static const void* split256_by_in(int in_dt, int out_dt) {
 template <int TM, int LW>
 static const void* logits_by_in(int in_dt) {
   switch (in_dt) {
+    case DT_F32:
+      if constexpr (TM == 128 && LW == 1) return tile_kernel_ptr<DT_F32, DT_F32, kEpiLogits, TM, LW>();
+      return nullptr;
     case DT_F16: return tile_kernel_ptr<DT_F16, DT_F32, kEpiLogits, TM, LW>();
     case DT_BF16: return tile_kernel_ptr<DT_BF16, DT_F32, kEpiLogits, TM, LW>();
     case DT_FP8: return tile_kernel_ptr<DT_FP8, DT_F32, kEpiLogits, TM, LW>();
@@ -1322,6 +1443,10 @@ const void* chain_kernel_symbol(int in_dt, int out_dt, int epi, int tile_rows, i
     if (epi == kEpiSplit) return split256_by_in(in_dt, out_dt);
     if (epi == kEpiLogits) return out_dt == DT_F32 ? logits_by_in<256, 0>(in_dt) : nullptr;
     return nullptr;
+  }
+  if (tile_rows == 64) {  // f32, exchange
+    if (in_dt != DT_F32 || epi != kEpiExchange) return nullptr;
+    return loaders ? by_out<DT_F32, kEpiExchange, 64, 1>(out_dt) : by_out<DT_F32, kEpiExchange, 64, 0>(out_dt);
   }
   if (tile_rows != 128) return nullptr;
   if (loaders) {
@@ -1347,40 +1472,39 @@ const void* rescale_kernel_symbol(int out_dt) {
 
 const void* zero_kernel_symbol() { return reinterpret_cast<const void*>(&zero_words_kernel); }
 
-template <int IN_DT, int LW>
+template <int IN_DT, int TM, int LW>
 static int lds_bytes_for(int out_dt) {
   switch (out_dt) {
-    case DT_F32: return EpiLayout<IN_DT, DT_F32, 128, LW, true>::TOTAL;
-    case DT_F16: return EpiLayout<IN_DT, DT_F16, 128, LW, true>::TOTAL;
-    case DT_BF16: return EpiLayout<IN_DT, DT_BF16, 128, LW, true>::TOTAL;
+    case DT_F32: return EpiLayout<IN_DT, DT_F32, TM, LW, true>::TOTAL;
+    case DT_F16: return EpiLayout<IN_DT, DT_F16, TM, LW, true>::TOTAL;
+    case DT_BF16: return EpiLayout<IN_DT, DT_BF16, TM, LW, true>::TOTAL;
   }
   return 0;
 }
 
-int chain_kernel_threads(int in_dt) {
-  switch (in_dt) {
-    case DT_F32: return Cfg<DT_F32>::kThreads;
-    case DT_F16: return Cfg<DT_F16>::kThreads;
-    case DT_BF16: return Cfg<DT_BF16>::kThreads;
-    case DT_FP8: return Cfg<DT_FP8>::kThreads;
-  }
-  return 0;
+int chain_kernel_threads(int in_dt, int tile_rows, int loaders) {
+  if (in_dt != DT_F32) return Cfg<DT_F16>::kThreads;
+  if (tile_rows == 64 && !loaders) return Cfg<DT_F32, 64, 0>::kThreads;
+  return Cfg<DT_F32, 128, 1>::kThreads;
 }
 
-int chain_kernel_lds_bytes(int in_dt, int out_dt, int loaders) {
+int chain_kernel_lds_bytes(int in_dt, int out_dt, int tile_rows, int loaders) {
+  if (in_dt == DT_F32) {
+    if (tile_rows == 64) return loaders ? lds_bytes_for<DT_F32, 64, 1>(out_dt) : lds_bytes_for<DT_F32, 64, 0>(out_dt);
+    return lds_bytes_for<DT_F32, 128, 1>(out_dt);
+  }
   if (loaders) {
     switch (in_dt) {
-      case DT_F16: return lds_bytes_for<DT_F16, 1>(out_dt);
-      case DT_BF16: return lds_bytes_for<DT_BF16, 1>(out_dt);
-      case DT_FP8: return lds_bytes_for<DT_FP8, 1>(out_dt);
+      case DT_F16: return lds_bytes_for<DT_F16, 128, 1>(out_dt);
+      case DT_BF16: return lds_bytes_for<DT_BF16, 128, 1>(out_dt);
+      case DT_FP8: return lds_bytes_for<DT_FP8, 128, 1>(out_dt);
     }
     return 0;
   }
   switch (in_dt) {
-    case DT_F32: return lds_bytes_for<DT_F32, 0>(out_dt);
-    case DT_F16: return lds_bytes_for<DT_F16, 0>(out_dt);
-    case DT_BF16: return lds_bytes_for<DT_BF16, 0>(out_dt);
-    case DT_FP8: return lds_bytes_for<DT_FP8, 0>(out_dt);
+    case DT_F16: return lds_bytes_for<DT_F16, 128, 0>(out_dt);
+    case DT_BF16: return lds_bytes_for<DT_BF16, 128, 0>(out_dt);
+    case DT_FP8: return lds_bytes_for<DT_FP8, 128, 0>(out_dt);
   }
   return 0;
 }

@@ -38,11 +38,12 @@ int device_cu_count(int fallback) {
   return prop.multiProcessorCount;
 }
 
-// Dynamic LDS added to an exchange kernel (wave layout `ks`) so that no CU
-// holds two of its workgroups (spreads a grid of <= CU-count tiles over all
-// CUs).
-int exchange_lds_pad(int in_dt, int out_dt, int loaders) {
-  const int stat = chain_kernel_lds_bytes(in_dt, out_dt, loaders);
+// Dynamic LDS added to an exchange kernel (its tile `ts`) so that no CU holds
+// two of its workgroups (spreads a grid of <= CU-count tiles over all CUs);
+// none when the grid needs a second one per CU.
+int exchange_lds_pad(int in_dt, int out_dt, const TileShape& ts, int64_t grid, int cu_count) {
+  if (ts.per_cu > 1 && grid > cu_count) return 0;
+  const int stat = chain_kernel_lds_bytes(in_dt, out_dt, ts.rows, ts.loaders);
   const int want = 80 * 1024 + 1024;
   return stat >= want ? 0 : want - stat;
 }
@@ -108,14 +109,18 @@ struct WsLayout {
   int64_t total;
 };
 
-WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int path) {
+WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int path) {
   WsLayout w{};
   const int64_t nT = ceil_div(n, kTile);
   w.gen_off = kGenOff;
   w.stats_off = align256(kGenOff + kGenBytes);
   // split statistics rows padded to 256 per batch (either tile height)
   const int64_t split_bytes = batch * ceil_div(m, 256) * 256 * nT * 8;
-  const int64_t exch_bytes = batch * ceil_div(m, kTile) * nT * kTile * 8;
+  int64_t exch_bytes = batch * ceil_div(m, kTile) * nT * kTile * 8;
+  if (in_dt == DT_F32) {  // 64 x 64 tiles, when the exchange path runs them: a slot each
+    const int64_t tiles = batch * ceil_div(m, 64) * ceil_div(n, 64);
+    if (tiles <= kMaxExchangeTiles && tiles * kTile * 8 > exch_bytes) exch_bytes = tiles * kTile * 8;
+  }
   w.stats_bytes = align256(split_bytes > exch_bytes ? split_bytes : exch_bytes);
   w.total = w.stats_off + w.stats_bytes;
   if (path == WTC_PATH_UNFUSED) {
@@ -149,6 +154,7 @@ int check_args(int64_t batch, int64_t m, int64_t n, int64_t k, int in_dt, int ou
 struct Plan {
   VariantDesc v{};
   int path = 0;
+  TileShape ts{};
   int64_t grid = 0, ws = 0;
   double est_us = 0;
 };
@@ -199,8 +205,9 @@ int plan_impl(int64_t batch, int64_t m, int64_t n, int64_t k, int in_dt, int out
   if (grid > 0x7FFFFFFFll) return fail(WTC_ERR_UNSUPPORTED, "too many tiles for one grid");
   out->v = c.v;
   out->path = c.path;
+  out->ts = tile_shape(c.v, c.path, pr);
   out->grid = grid;
-  out->ws = ws_layout(batch, m, n, c.path).total;
+  out->ws = ws_layout(batch, m, n, in_dt, c.path).total;
   out->est_us = c.est_us;
   return WTC_OK;
 }
@@ -316,13 +323,21 @@ int device_state(int dev, DeviceState** out, bool host_objects = true) {
       for (int o = 0; o < 3; ++o) {
         s.occ[i][o] = 1 << 30;
         for (int lw = 0; lw <= 1; ++lw) {
-          const void* fn = chain_kernel_symbol(i, o, kEpiExchange, 128, lw);
-          if (!fn) continue;  // f32 has no loader-wave layout
-          const int pad = exchange_lds_pad(i, o, lw);
-          HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, pad));
-          int nb = 0;
-          HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, chain_kernel_threads(i), pad));
-          if (nb < s.occ[i][o]) s.occ[i][o] = nb;
+          if (const void* fn = chain_kernel_symbol(i, o, kEpiExchange, 128, lw)) {
+            const int pad = exchange_lds_pad(i, o, {128, 128, lw, 1}, 0, s.cu_count);
+            HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, pad));
+            int nb = 0;
+            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, chain_kernel_threads(i, 128, lw), pad));
+            if (nb < s.occ[i][o]) s.occ[i][o] = nb;
+          }
+          if (const void* fn = chain_kernel_symbol(i, o, kEpiExchange, 64, lw)) {  // f32
+            const int pad = exchange_lds_pad(i, o, {64, 64, lw, 1}, 0, s.cu_count);
+            HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, pad));
+            int nb = 0;
+            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, chain_kernel_threads(i, 64, lw), 0));
+            if (nb < kF32SmallTilesPerCu)
+              return fail(WTC_ERR_HIP, "a CU holds fewer 64 x 64 tiles than the launch plan counts on");
+          }
         }
       }
     s.init = true;
@@ -410,9 +425,10 @@ struct TileKernel {
   const void* fn;
   int threads;
 };
-TileKernel tile_kernel(const VariantDesc& v, int in_dt, int out_dt, int epi) {
+TileKernel tile_kernel(const VariantDesc& v, const TileShape& ts, int in_dt, int out_dt, int epi) {
   if (v.id == kVarTile256x256) return {wide_kernel_symbol(in_dt, out_dt, epi), wide_kernel_threads()};
-  return {chain_kernel_symbol(in_dt, out_dt, epi, v.tile_rows, v.loaders), chain_kernel_threads(in_dt)};
+  return {chain_kernel_symbol(in_dt, out_dt, epi, ts.rows, ts.loaders),
+          chain_kernel_threads(in_dt, ts.rows, ts.loaders)};
 }
 
 // chain_tile_kernel: the scalars a tile needs before its first load lead the
@@ -729,7 +745,7 @@ int64_t wtc_matmul_softmax_workspace_size(int64_t batch, int64_t m, int64_t n, i
                                           int in_dtype, int out_dtype, int path) {
   g_last_error.clear();
   if (check_args(batch, m, n, k, in_dtype, out_dtype, path)) return -1;
-  return ws_layout(batch, m, n, path).total;
+  return ws_layout(batch, m, n, in_dtype, path).total;
 }
 
 int wtc_workspace_init(void* workspace, size_t workspace_bytes, void* stream) {
@@ -902,7 +918,7 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
     rc = default_workspace(ds, need, &ws, stream);
     if (rc) return rc;
   }
-  const WsLayout L = ws_layout(batch, m, n, chosen);
+  const WsLayout L = ws_layout(batch, m, n, in_dtype, chosen);
   uint8_t* wsb = static_cast<uint8_t*>(ws);
 
   const int isz = dtype_bytes(in_dtype), osz = dtype_bytes(out_dtype);
@@ -923,10 +939,9 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
   p.c2 = lin * 1.4426950408889634f;
   p.lin_scale = lin;
   // row blocks per batch of the kernel that runs
-  const int tile_rows = var.tile_rows;
+  const int tile_rows = pl.ts.rows;
   p.nRB = (int)ceil_div(m, tile_rows);
-  // column tiles per row block: the variant's on the split and unfused paths
-  p.nT = (int)ceil_div(n, chosen == WTC_PATH_SPLIT || chosen == WTC_PATH_UNFUSED ? var.tile_n : kTile);
+  p.nT = (int)ceil_div(n, pl.ts.cols);  // column tiles per row block
   p.partial = reinterpret_cast<float2*>(wsb + L.stats_off);
   p.ent = reinterpret_cast<uint64_t*>(wsb + L.stats_off);
   p.gen = reinterpret_cast<uint32_t*>(wsb + L.gen_off);
@@ -941,11 +956,11 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
                         p, stream);
   }
   if (chosen == WTC_PATH_EXCHANGE)
-    return launch_exchange(ds, chain_kernel_symbol(in_dtype, out_dtype, kEpiExchange, 128, var.loaders),
-                           chain_kernel_threads(in_dtype), grid,
-                           exchange_lds_pad(in_dtype, out_dtype, var.loaders), p, stream);
+    return launch_exchange(ds, chain_kernel_symbol(in_dtype, out_dtype, kEpiExchange, pl.ts.rows, pl.ts.loaders),
+                           chain_kernel_threads(in_dtype, pl.ts.rows, pl.ts.loaders), grid,
+                           exchange_lds_pad(in_dtype, out_dtype, pl.ts, grid, cu_count), p, stream);
   if (chosen == WTC_PATH_SPLIT) {
-    const TileKernel tk = tile_kernel(var, in_dtype, out_dtype, kEpiSplit);
+    const TileKernel tk = tile_kernel(var, pl.ts, in_dtype, out_dtype, kEpiSplit);
     rc = launch_tile(tk.fn, tk.threads, grid, 0, p, stream);
     if (rc) return rc;
     uint8_t* o = p.out;
@@ -970,7 +985,7 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
   q.out = reinterpret_cast<uint8_t*>(logits);
   q.o_bstride = m * n * 4;
   q.ldo_bytes = n * 4;
-  const TileKernel tk = tile_kernel(var, in_dtype, DT_F32, kEpiLogits);
+  const TileKernel tk = tile_kernel(var, pl.ts, in_dtype, DT_F32, kEpiLogits);
   rc = launch_tile(tk.fn, tk.threads, grid, 0, q, stream);
   if (rc) return rc;
   const int64_t rows = batch * m;

@@ -186,6 +186,13 @@ WTC_HD constexpr int dma64_a_row(int b, int lane) { return 16 * b + (lane >> 2);
 WTC_HD constexpr int dma64_a_chunk(int b, int lane) {
   return (lane & 3) ^ ((dma64_a_row(b, lane) >> 2) & 3);
 }
+// f32 64 x 64 tiles: a bf16 plane of B, [32 k-rows][64 columns], K-major with
+// 128 bytes per k-row, its halves swapped by (k / 2) % 2: the four k-rows of a
+// 16-lane transpose read (64 bytes of each over two lane groups) then fall in
+// distinct banks.
+WTC_HD constexpr int f32_btr64_offset(int k, int n) {
+  return k * 128 + ((((n >> 3) ^ (((k >> 1) & 1) << 2)) & 7) << 4) + (n & 7) * 2;
+}
 // MFMA A fragments from a k-slab: 16-bit k-step s (0, 1) takes chunk
 // 2s + lane/32 of row lane%32; fp8 (one k-step of 64) takes chunks
 // 2*(lane/32) + hh, hh = 0, 1.

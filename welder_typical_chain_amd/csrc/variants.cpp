@@ -35,31 +35,31 @@ constexpr unsigned kSplitPaths = bit(WTC_PATH_SPLIT) | bit(WTC_PATH_UNFUSED);
 // The constants were fitted (least squares on the log of the time) to
 // back-to-back timings of every variant on every path over the 60 shapes
 // of calibrate.py on MI355X.  Fitted on three of its four shape sets and
-// scored on the fourth, in turn, the fused ranking lost 0.84 % on average
+// scored on the fourth, in turn, the fused ranking lost 0.89 % on average
 // against the measured fastest choice (the hand-written rules it replaces:
 // 5.3 %).
 struct TileCal {
   double kt_cyc;        // own cycles per k-tile
   double fixed_cyc[3];  // per tile: exchange, split, logits epilogues
 };
-// [tile variant][0: 16-bit, 1: fp8, 2: f32]; fixed parts shared across input
-// types.  Rows: kVarTile128, kVarTile128Loaders, kVarTile256, kVarTile256x256.
-const TileCal kTileCal[4][3] = {
-    /* kVarTile128 */ {{635.87, {3678.9, 5946.6, 0}}, {617.19, {3678.9, 5946.6, 0}}, {4521.3, {3678.9, 5946.6, 0}}},
-    /* kVarTile128Loaders */ {{562.07, {4068.6, 6487.6, 254}}, {530.85, {4068.6, 6487.6, 254}}, {0, {0, 0, 0}}},
-    /* kVarTile256 */ {{1142.1, {0, 11628.2, 0}}, {1286.6, {0, 11628.2, 0}}, {0, {0, 0, 0}}},
-    /* kVarTile256x256 */ {{1973.6, {0, 20944.0, 6164}}, {1635.5, {0, 20944.0, 6164}}, {0, {0, 0, 0}}},
+// [tile variant][0: 16-bit, 1: fp8, 2: f32, 3: f32 64 x 64]; fixed parts shared
+// across 16-bit and fp8 inputs.  Rows: kVarTile128, kVarTile128Loaders, kVarTile256, kVarTile256x256.
+const TileCal kTileCal[4][4] = {
+    /* kVarTile128 */ {{631.76, {3378.7, 5839.9, 0}}, {612.52, {3378.7, 5839.9, 0}}, {2176.7, {4720.4, 6778.6, 0}}, {565.57, {5245.6, 0, 0}}},
+    /* kVarTile128Loaders */ {{558.27, {3771.6, 6373.3, 254}}, {526.47, {3771.6, 6373.3, 254}}, {0, {0, 0, 0}}},
+    /* kVarTile256 */ {{1139.2, {0, 11392.3, 0}}, {1283.0, {0, 11392.3, 0}}, {0, {0, 0, 0}}},
+    /* kVarTile256x256 */ {{1971.5, {0, 20552.0, 6164}}, {1633.1, {0, 20552.0, 6164}}, {0, {0, 0, 0}}},
 };
 int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // Rows kernel, cycles per row block: a fixed part, and per 128-column tile
 // (both passes) a fixed part and a part per 16-wide k-step.
-constexpr double kRowsBlockCyc = 1983.1, kRowsTileCyc = 4932.5, kRowsKstepCyc = 102.19;
+constexpr double kRowsBlockCyc = 1939.3, kRowsTileCyc = 4930.8, kRowsKstepCyc = 102.65;
 // Back-to-back launch cost of one kernel (us); the row exchange after the
 // last tile of a row block: fixed (us) and per column tile (us); the HBM
 // rate of the fused paths' streaming passes and the chip-wide rate that
 // prices k-tile bytes (GB/s).
-constexpr double kLaunchUs = 3.6597, kExchangeUs = 0.2592, kExchangePerTileUs = 0.08580;
-constexpr double kHbmGBs = 7919.8, kFeedGBs = 83312.1;
+constexpr double kLaunchUs = 3.6813, kExchangeUs = 0.3895, kExchangePerTileUs = 0.09190;
+constexpr double kHbmGBs = 7664.6, kFeedGBs = 81910.8;
 // Unfused row passes (one 256-thread workgroup per row, eight per CU): HBM
 // rate, and the rate one workgroup streams its row at (GB/s).
 constexpr double kRowPassHbmGBs = 5293.0, kRowPassWgGBs = 5.573;
@@ -144,6 +144,19 @@ bool feasible(const VariantDesc& v, int path, const Problem& p) {
   }
 }
 
+TileShape tile_shape(const VariantDesc& v, int path, const Problem& p) {
+  if (path == WTC_PATH_ROWS) return {128, 128, 0, 1};
+  if (p.in_dt != WTC_DTYPE_F32)
+    return {v.tile_rows, (int)v.tile_n, v.loaders, path == WTC_PATH_EXCHANGE ? std::max(1, p.xch_per_cu) : 1};
+  if (path == WTC_PATH_EXCHANGE) {
+    const int64_t nT = cdiv(p.n, 64), tiles = p.batch * cdiv(p.m, 64) * nT;
+    if (tiles <= (int64_t)kF32SmallTilesPerCu * p.cu_count && tiles <= kExchangeMaxTiles &&
+        nT <= kExchangeMaxColTiles)
+      return {64, 64, p.k > kF32OneGroupK ? 1 : 0, kF32SmallTilesPerCu};
+  }
+  return {128, 128, 1, 1};
+}
+
 std::string infeasible_reason(const VariantDesc& v, int path, const Problem& p) {
   static const char* const kPathNames[] = {"auto", "exchange", "split", "unfused", "rows"};
   if (path < WTC_PATH_EXCHANGE || path > WTC_PATH_ROWS) return "unknown path";
@@ -178,7 +191,8 @@ std::string infeasible_reason(const VariantDesc& v, int path, const Problem& p) 
 
 int64_t variant_grid(const VariantDesc& v, int path, const Problem& p) {
   if (path == WTC_PATH_ROWS) return p.batch * cdiv(p.m, 128);
-  return p.batch * cdiv(p.m, v.tile_rows) * cdiv(p.n, v.tile_n);
+  const TileShape ts = tile_shape(v, path, p);
+  return p.batch * cdiv(p.m, ts.rows) * cdiv(p.n, ts.cols);
 }
 
 double estimate_us(const VariantDesc& v, int path, const Problem& p) {
@@ -187,7 +201,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
   const double elems = (double)p.batch * (double)p.m * (double)p.n;
   const double ab_bytes = (double)p.batch * ((double)p.m * p.k + (double)p.k * p.n) * isz;
   const double us_per_byte = 1e6 / (kHbmGBs * 1e9);
-  const double nT = (double)cdiv(p.n, path == WTC_PATH_ROWS ? 128 : v.tile_n);
+  const TileShape ts = tile_shape(v, path, p);
+  const double nT = (double)cdiv(p.n, ts.cols);
   if (path == WTC_PATH_ROWS) {
     const double blocks = (double)variant_grid(v, path, p);
     const double waves = std::ceil(blocks / cu);
@@ -197,13 +212,13 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
     return kLaunchUs + std::max(t_blocks, t_hbm);
   }
-  const TileCal& cal = kTileCal[cal_row(v.id)][in_class(p.in_dt)];
+  const TileCal& cal = kTileCal[cal_row(v.id)][in_class(p.in_dt) + (ts.rows == 64 ? 1 : 0)];
   const int epi = path == WTC_PATH_EXCHANGE ? 0 : (path == WTC_PATH_SPLIT ? 1 : 2);
   const double tiles = (double)variant_grid(v, path, p);
   const double waves = std::ceil(tiles / cu);
   const double f = clock_ghz(tiles / (waves * cu));
   const double nk = (double)cdiv(p.k * in_bytes(p.in_dt), 128);
-  const double kt_bytes = (double)(v.tile_rows + v.tile_n) * 128.0;  // A and B per 128 bytes of K
+  const double kt_bytes = (double)(ts.rows + ts.cols) * 128.0;  // A and B per 128 bytes of K
   auto wave_us = [&](double active) {
     const double kt = cal.kt_cyc + kt_bytes * active * f / kFeedGBs;
     return (cal.fixed_cyc[epi] + nk * kt) / (f * 1e3);
@@ -212,7 +227,7 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
   const double t_tiles = full * wave_us(cu) + (rem > 0 ? wave_us(rem) : 0.0);
   if (path == WTC_PATH_EXCHANGE) {
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
-    const double t_xch = p.n > 128 ? kExchangeUs + kExchangePerTileUs * nT : 0.0;
+    const double t_xch = p.n > ts.cols ? kExchangeUs + kExchangePerTileUs * nT : 0.0;
     return kLaunchUs + std::max(t_tiles, t_hbm) + t_xch;
   }
   if (path == WTC_PATH_SPLIT) {

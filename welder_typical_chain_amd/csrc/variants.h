@@ -64,6 +64,21 @@ struct Problem {
   int xch_per_cu; // exchange-kernel workgroups one CU holds (1 with its LDS pad)
 };
 
+// The tile that a variant's first kernel runs a problem with.
+struct TileShape {
+  int rows, cols;
+  int loaders;  // loader waves (f32: two k-groups)
+  int per_cu;   // workgroups a CU holds at once on the exchange path
+};
+// The variant's own tile, except for f32 on the exchange path: 64 x 64 tiles
+// (instead of 128 x 128) while two of them per CU hold the whole problem, since
+// f32 tiles are bound by their own CU's arithmetic and a 128-row grid would
+// leave CUs without one (1024 x 1024 x 1024: 64 tiles of 128 rows, 256 of 64).
+// Short K (up to kF32OneGroupK): one k-group, whose sums need not meet.
+constexpr int kF32SmallTilesPerCu = 2;
+constexpr int64_t kF32OneGroupK = 192;
+TileShape tile_shape(const VariantDesc& v, int path, const Problem& p);
+
 // Whether a (variant, path) pair can run a problem, and why not (empty when
 // it can; builds the message, so only for error reports).
 bool feasible(const VariantDesc& v, int path, const Problem& p);

@@ -24,8 +24,8 @@ struct ChainParams {
   int64_t lda_bytes, ldb_bytes, ldo_bytes;  // row pitches in bytes
   float c2;         // scale * log2(e): softmax runs as exp2(c2*x - max)
   float lin_scale;  // scale for kEpiLogits
-  int nRB;          // row blocks (of 128 rows) per batch
-  int nT;           // column tiles (of 128 columns) per row block
+  int nRB;          // row blocks (of the tile's rows) per batch
+  int nT;           // column tiles (of the tile's columns) per row block
   float2* partial;  // split path: [batch][nRB * tile rows][nT] per-tile row (max, sumexp), log2
   uint64_t* ent;    // exchange path: [slot][128] tagged per-row log-sum-exp entries
   uint32_t* gen;    // exchange path: [kMaxExchangeTiles] slot generation words
@@ -35,18 +35,20 @@ struct ChainParams {
   uint64_t spin_ticks;  // exchange wait limit, 100 MHz ticks
 };
 
-// tile_rows: 128, or 256 (split epilogue, and f32 logits, with 16-bit or fp8
-// inputs); loaders: 1 for the 128-row layout with 4 MFMA and 4 loader waves
-// (exchange and split epilogues, and f32 logits, with 16-bit or fp8 inputs).
-// NULL for a combination not built.
-const void* chain_kernel_symbol(int in_dt, int out_dt, int epi, int tile_rows = 128, int loaders = 0);
+// 16-bit and fp8 inputs: 128-column tiles; tile_rows: 128, or 256 (split
+// epilogue, and f32 logits); loaders: 1 for the 128-row layout with 4 MFMA and
+// 4 loader waves (exchange and split epilogues, and f32 logits).  f32 inputs:
+// tile_rows 128 (128 x 128, loaders = 1: two k-groups) or, exchange epilogue,
+// 64 (64 x 64, one or two k-groups).  NULL for a combination not built.
+const void* chain_kernel_symbol(int in_dt, int out_dt, int epi, int tile_rows, int loaders);
 const void* rescale_kernel_symbol(int out_dt);
 // Waves that share one row in rescale_rows_kernel (its grid is rows * wpr / 4).
 int rescale_waves_per_row(int64_t rows_total, int cu_count);
 const void* zero_kernel_symbol();
-// Static LDS of the exchange-epilogue kernel of this wave layout.
-int chain_kernel_lds_bytes(int in_dt, int out_dt, int loaders = 0);
-int chain_kernel_threads(int in_dt);  // workgroup size of chain_tile_kernel (every layout)
+// Static LDS of the exchange-epilogue kernel of this layout, and the workgroup
+// size of the layout's kernels (every epilogue).
+int chain_kernel_lds_bytes(int in_dt, int out_dt, int tile_rows, int loaders);
+int chain_kernel_threads(int in_dt, int tile_rows, int loaders);
 
 // 256x256 tiles (wide_tile.hip): split epilogue (any output type) or f32
 // logits, 16-bit or fp8 inputs; NULL otherwise.  Same arguments as
