@@ -27,6 +27,7 @@ namespace wtc {
 int chain_kernel_threads(int in_dt, int tile_rows, int loaders);
 int wide_kernel_threads();
 int rows_kernel_threads();
+int few_rows_kernel_threads();
 int rescale_waves_per_row(int64_t rows_total, int cu_count);
 // Compute units of the current device, or `fallback` when no GPU is visible.
 int device_cu_count(int fallback);
@@ -188,6 +189,17 @@ static std::string emit_loop_structure(const ChainSpec& spec, const VariantDesc&
            "direct-to-LDS ring\n"
         << "          scf.for %s = %c0 to %ks step %c1 {  // " << mfma << "\n          }\n"
         << "        }\n      }\n";
+    } else if (k.kind == "few_rows") {
+      c("nT", (spec.n + 127) / 128);
+      c("ks", (spec.k + 15) / 16);
+      c("m", spec.m);
+      c("n", spec.n);
+      o << "      // one batch: all rows and columns, logits in LDS\n"
+        << "      scf.for %t = %c0 to %nT step %c1 {  // 128-column B tiles, read once through a "
+           "direct-to-LDS ring\n"
+        << "        scf.for %s = %c0 to %ks step %c1 {  // " << mfma << "\n        }\n      }\n"
+        << "      scf.for %r = %c0 to %m step %c1 {  // row max, exp2, sum, product\n"
+        << "        scf.for %j = %c0 to %n step %c1 {\n        }\n      }\n";
     } else if (k.kind == "rescale") {
       c("n", spec.n);
       c("nT", nT);
@@ -314,7 +326,13 @@ static int compile_impl(const char* input_mlir_path, const char* out_dir, int64_
   std::vector<K> ks;
   const int64_t rows = spec.batch * spec.m;
   const int tile_threads = wide ? wide_kernel_threads() : chain_kernel_threads(in_code, ts.rows, ts.loaders);
-  if (path == WTC_PATH_ROWS) {
+  if (path == WTC_PATH_ROWS && ts.rows == kFewRows) {
+    const char* stages = ts.per_cu == 2 ? "4" : "6";
+    ks.push_back({"chain_few_rows_kernel<" + kin + "," + kout + "," + stages + " stages>",
+                  "_ZN3wtc21chain_few_rows_kernelILi" + std::to_string(in_code) + "ELi" +
+                      std::to_string(out_code) + "ELi" + stages + "E",
+                  grid, 0, few_rows_kernel_threads(), "few_rows"});
+  } else if (path == WTC_PATH_ROWS) {
     ks.push_back({"chain_rows_kernel<" + kin + "," + kout + ">",
                   "_ZN3wtc17chain_rows_kernelILi" + std::to_string(in_code) + "ELi" +
                       std::to_string(out_code) + "E",

@@ -49,6 +49,8 @@ int exchange_lds_pad(int in_dt, int out_dt, const TileShape& ts, int64_t grid, i
 }
 
 static_assert(kExchangeMaxTiles == kMaxExchangeTiles, "exchange slot limit");
+static_assert(kFewRowsLogits == kFewRowsMaxLogits && kFewRowsLogitsPair == kFewRowsPairLogits && kFewRowsPad == 4,
+              "few-row kernel limits");
 }  // namespace wtc
 
 namespace {
@@ -951,6 +953,10 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
 
   const int cu_count = ds->cu_count;
   if (chosen != WTC_PATH_EXCHANGE) lk.unlock();
+  if (chosen == WTC_PATH_ROWS && pl.ts.rows == kFewRows) {
+    return launch_chain(few_rows_kernel_symbol(in_dtype, out_dtype, pl.ts.per_cu == 2 ? 4 : 6),
+                        few_rows_kernel_threads(), grid, 0, p, stream);
+  }
   if (chosen == WTC_PATH_ROWS) {
     return launch_chain(rows_kernel_symbol(in_dtype, out_dtype), rows_kernel_threads(), grid, 0,
                         p, stream);

@@ -54,6 +54,14 @@ int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // Rows kernel, cycles per row block: a fixed part, and per 128-column tile
 // (both passes) a fixed part and a part per 16-wide k-step.
 constexpr double kRowsBlockCyc = 1939.3, kRowsTileCyc = 4930.8, kRowsKstepCyc = 102.65;
+// Few-row kernel: a workgroup's first loads and its softmax (us), one 16 KiB unit
+// of B (us), and the rate at which all workgroups together read B (GB/s): read
+// off 36 timings of 4 to 512 batches x 1 to 16 rows x 256 to 7936 columns (not
+// in the table above, whose shapes have more rows).  For so few rows the model
+// prices the 128-row tiles up to a quarter too high, so the few-row kernel is
+// priced a quarter too high as well: it then lost nowhere against them (16 x 1 x
+// 2304 x 128: 13.8 us, split 11.7; 32 x 2 x 1312 x 128: 10.5 and 12.1).
+constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFewMargin = 1.25;
 // Back-to-back launch cost of one kernel (us); the row exchange after the
 // last tile of a row block: fixed (us) and per column tile (us); the HBM
 // rate of the fused paths' streaming passes and the chip-wide rate that
@@ -145,7 +153,11 @@ bool feasible(const VariantDesc& v, int path, const Problem& p) {
 }
 
 TileShape tile_shape(const VariantDesc& v, int path, const Problem& p) {
-  if (path == WTC_PATH_ROWS) return {128, 128, 0, 1};
+  if (path == WTC_PATH_ROWS) {
+    const int64_t logits = p.m * (cdiv(p.n, 128) * 128 + 4);
+    if (p.m > kFewRows || logits > kFewRowsLogits) return {128, 128, 0, 1};
+    return {(int)kFewRows, 128, 0, logits <= kFewRowsLogitsPair && p.batch > p.cu_count ? 2 : 1};
+  }
   if (p.in_dt != WTC_DTYPE_F32)
     return {v.tile_rows, (int)v.tile_n, v.loaders, path == WTC_PATH_EXCHANGE ? std::max(1, p.xch_per_cu) : 1};
   if (path == WTC_PATH_EXCHANGE) {
@@ -190,9 +202,9 @@ std::string infeasible_reason(const VariantDesc& v, int path, const Problem& p) 
 }
 
 int64_t variant_grid(const VariantDesc& v, int path, const Problem& p) {
-  if (path == WTC_PATH_ROWS) return p.batch * cdiv(p.m, 128);
   const TileShape ts = tile_shape(v, path, p);
-  return p.batch * cdiv(p.m, ts.rows) * cdiv(p.n, ts.cols);
+  const int64_t row_blocks = p.batch * cdiv(p.m, ts.rows);
+  return path == WTC_PATH_ROWS ? row_blocks : row_blocks * cdiv(p.n, ts.cols);  // rows: all of n per workgroup
 }
 
 double estimate_us(const VariantDesc& v, int path, const Problem& p) {
@@ -205,6 +217,16 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
   const double nT = (double)cdiv(p.n, ts.cols);
   if (path == WTC_PATH_ROWS) {
     const double blocks = (double)variant_grid(v, path, p);
+    if (ts.rows == kFewRows) {
+      // one stream of B per batch: 16 KiB units at what a CU's loads in flight
+      // bring, or at the HBM rate shared with the other workgroups
+      const double units = nT * (p.k > 64 ? 2 : 1);
+      auto round_us = [&](double active) {
+        return kFewFixedUs / ts.per_cu + std::max(units * kFewUnitUs, ab_bytes / blocks * active * 1e6 / (kFewHbmGBs * 1e9));
+      };
+      const double full = std::floor(blocks / cu), rem = blocks - full * cu;
+      return kFewMargin * (kLaunchUs + full * round_us(cu) + (rem > 0 ? round_us(rem) : 0.0));
+    }
     const double waves = std::ceil(blocks / cu);
     const double f = clock_ghz(blocks / (waves * cu));
     const double cyc = kRowsBlockCyc + nT * (kRowsTileCyc + kRowsKstepCyc * (double)cdiv(p.k, 16));

@@ -68,7 +68,7 @@ struct Problem {
 struct TileShape {
   int rows, cols;
   int loaders;  // loader waves (f32: two k-groups)
-  int per_cu;   // workgroups a CU holds at once on the exchange path
+  int per_cu;   // workgroups a CU holds at once (exchange path, few-row kernel)
 };
 // The variant's own tile, except for f32 on the exchange path: 64 x 64 tiles
 // (instead of 128 x 128) while two of them per CU hold the whole problem, since
@@ -77,6 +77,12 @@ struct TileShape {
 // Short K (up to kF32OneGroupK): one k-group, whose sums need not meet.
 constexpr int kF32SmallTilesPerCu = 2;
 constexpr int64_t kF32OneGroupK = 192;
+// And on the rows path: one 32-row block per batch (chain_few_rows_kernel, which
+// reads B once) when the problem has at most that many rows and their logits fit
+// in LDS, kFewRowsLogits floats with each row's columns padded to 128 + 4; two
+// workgroups per CU when they fit a quarter of that and the batches outnumber
+// the CUs.
+constexpr int64_t kFewRows = 32, kFewRowsLogits = 16384, kFewRowsLogitsPair = 4096;
 TileShape tile_shape(const VariantDesc& v, int path, const Problem& p);
 
 // Whether a (variant, path) pair can run a problem, and why not (empty when

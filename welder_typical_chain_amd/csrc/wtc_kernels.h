@@ -62,6 +62,14 @@ const void* rows_kernel_symbol(int in_dt, int out_dt);
 int rows_kernel_threads();
 int rows_kernel_max_k();
 
+// One workgroup per batch of few rows (tile_shape's rule: rows, logits that fit
+// LDS); `stages`: 6, or 4 for two workgroups per CU.
+constexpr int kFewRowsMaxLogits = 16384;  // floats of logits a workgroup keeps
+constexpr int kFewRowsPairLogits = 4096;  // ... with two workgroups per CU
+constexpr int kFewRowsPad = 4;            // floats after each row: rows start in different banks
+const void* few_rows_kernel_symbol(int in_dt, int out_dt, int stages);
+int few_rows_kernel_threads();
+
 // Unfused five-kernel baseline (matmul, row max, exp, row sum, divide).
 const void* rowmax_kernel_symbol();
 const void* expsub_kernel_symbol();
