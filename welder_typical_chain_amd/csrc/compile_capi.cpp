@@ -335,7 +335,7 @@ static int compile_impl(const char* input_mlir_path, const char* out_dir, int64_
   } else if (path == WTC_PATH_ROWS) {
     ks.push_back({"chain_rows_kernel<" + kin + "," + kout + ">",
                   "_ZN3wtc17chain_rows_kernelILi" + std::to_string(in_code) + "ELi" +
-                      std::to_string(out_code) + "E",
+                      std::to_string(out_code) + "ELi" + (spec.k <= 64 ? "4" : "8") + "E",
                   grid, 0, rows_kernel_threads(), "rows"});
   } else if (path == WTC_PATH_EXCHANGE) {
     const auto tk = tile_kern(out_code, kout, 0, "exchange");

@@ -958,7 +958,7 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
                         few_rows_kernel_threads(), grid, 0, p, stream);
   }
   if (chosen == WTC_PATH_ROWS) {
-    return launch_chain(rows_kernel_symbol(in_dtype, out_dtype), rows_kernel_threads(), grid, 0,
+    return launch_chain(rows_kernel_symbol(in_dtype, out_dtype, rows_ksteps(k)), rows_kernel_threads(), grid, 0,
                         p, stream);
   }
   if (chosen == WTC_PATH_EXCHANGE)

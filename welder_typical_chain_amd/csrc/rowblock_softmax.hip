@@ -11,9 +11,9 @@
 //   pass 2: the same products again, out = exp2(y - max) / sum, stored once.
 // The output is written exactly once and nothing else goes to HBM (no
 // workspace).  The row block's A goes to LDS once and its MFMA fragments stay
-// in registers for both passes; the B column tiles stream through a 3-stage
-// LDS ring of direct-to-LDS loads (the same K-major, XOR-swizzled B layout
-// and transpose reads as chain_tile_kernel).
+// in registers for both passes; the B column tiles stream through a
+// 3- or 4-stage LDS ring of direct-to-LDS loads (the same K-major, XOR-swizzled
+// B layout and transpose reads as chain_tile_kernel).
 //
 // 12 waves in two roles, three per SIMD:
 //   compute waves 0-7, 2 x 4: wave (wm, wn) owns rows wm*64 .. +63 and
@@ -45,25 +45,32 @@ namespace rows {
 
 constexpr int BM = 128;             // rows per workgroup
 constexpr int BN = 128;             // columns per tile
-constexpr int NCW = 8;             // compute waves, 2 x 4 (64 x 32 each)
+constexpr int NCW = 8;              // compute waves, 2 x 4 (64 x 32 each)
 constexpr int NT = 64 * (NCW + 4);  // threads: 8 compute waves, then 4 I/O waves
-constexpr int KS = 8;               // k-steps of 16: K <= 128
-constexpr int A_KT = KS / 4;        // A k-tiles of 64 elements (128 bytes) per row
-constexpr int A_BYTES = A_KT * BM * 128;  // the row block's A, 32 KiB
-constexpr int STAGE = KS * 16 * 256;  // one B tile, 128 k-rows x 256 bytes (32 KiB)
-constexpr int OUT_STAGE = BM * 256;   // one tile of 16-bit outputs (32 KiB)
-constexpr int S = 3;                // ring stages
-constexpr int OUT0 = 0;             // out stage 0: the A region, once A is in registers
-constexpr int OUT1 = A_BYTES;       // out stage 1, and the pass-1 statistics merge
+constexpr int OUT_STAGE = BM * 256;  // one tile of 16-bit outputs (32 KiB)
+constexpr int SPW = BM / 4 / 4;      // store instructions per I/O wave and tile (8)
+constexpr int OUT0 = 0;              // out stage 0: over the A region, once A is in registers
+constexpr int OUT1 = OUT_STAGE;      // out stage 1, and the pass-1 statistics merge
 constexpr int RING_OFF = OUT1 + OUT_STAGE;
-constexpr int BLK = STAGE / 1024;   // 1 KiB load blocks per B tile (32)
-constexpr int BPW = BLK / 4;        // B blocks per I/O wave (8)
-constexpr int ABPW = A_KT * 16 / 4;  // A blocks per I/O wave (8)
-constexpr int SPW = BM / 4 / 4;     // store instructions per I/O wave and tile (8)
-constexpr int LDS_BYTES = RING_OFF + S * STAGE;  // 160 KiB
-static_assert(LDS_BYTES <= 160 * 1024, "LDS");
-static_assert(A_BYTES == OUT_STAGE, "out stage 0 reuses the A region");
 static_assert(2 * 4 * BM * 4 <= OUT_STAGE, "row statistics fit in out stage 1");
+
+// KS k-steps of 16: 8 (K <= 128) or 4 (K <= 64, where the other half of the
+// MFMAs, fragment reads and tile bytes would be zeros).  Measured at K = 64, 8
+// against 4 k-steps (us a call): 64 x 1024 x 1024 50.5 -> 42.6, 32 x 2048 x 2048
+// 88.9 -> 78.9, 24 x 777 x 1000 26.95 -> 24.9; a ring of 3, 4, 5 or 6 stages
+// within 1 us of each other (43.8, 42.6, 42.6, 42.9 for the first).
+template <int KS> struct Geo {
+  static constexpr int A_KT = KS / 4;               // A k-tiles of 64 elements (128 bytes) per row
+  static constexpr int A_BYTES = A_KT * BM * 128;   // the row block's A
+  static constexpr int STAGE = KS * 16 * 256;       // one B tile, 16 KS k-rows x 256 bytes
+  static constexpr int BPW = STAGE / 1024 / 4;      // B load blocks per I/O wave and tile
+  static constexpr int ABPW = A_KT * 16 / 4;        // A blocks per I/O wave
+  static constexpr int KPG = KS / 4;                // k-steps per group of a phase
+  static constexpr int S = KS == 8 ? 3 : 4;         // ring stages
+  static constexpr int LDS_BYTES = RING_OFF + S * STAGE;
+  static_assert(KS % 4 == 0 && LDS_BYTES <= 160 * 1024, "LDS");
+  static_assert(A_BYTES <= OUT_STAGE, "out stage 0 reuses the A region");
+};
 
 // the out stage's layout: rows_out_offset (tile_layout.h)
 __device__ inline int out_offset(int r, int c) { return rows_out_offset(r, c); }
@@ -80,11 +87,13 @@ __device__ inline f32x16 mfma16(const u32x4& b, const u32x4& a, const f32x16& c)
                                                    __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
 }
 
-template <int IN_DT, int OUT_DT>
+template <int IN_DT, int OUT_DT, int KS>
 __global__ void __launch_bounds__(rows::NT, 1)
 chain_rows_kernel(const ChainParams p) {
   using namespace rows;
-  __shared__ __attribute__((aligned(16))) uint8_t smem[LDS_BYTES];
+  using G = Geo<KS>;
+  constexpr int STAGE = G::STAGE, BPW = G::BPW, ABPW = G::ABPW, KPG = G::KPG, S = G::S;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[G::LDS_BYTES];
 
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -165,42 +174,49 @@ chain_rows_kernel(const ChainParams p) {
         __builtin_amdgcn_raw_buffer_store_b128(x, ro, col < N ? (int)off : (int)kOutOfRange, 0, kCachePolicyNT);
       }
     };
-    // I/O step `it` (between B(it) and B(it+1)): the loads of tile it+S-1,
-    // BM where it falls, the stores of tile it-2 (ST), then the wait for
-    // tile it+1: issued in step it-1 (or the prologue), followed by the
-    // stores of step it-1 and this step's loads and stores -- vector memory
-    // operations of one wave complete in order.
-    auto iostep = [&](int it, auto st_c, auto wait_c, auto merge_c) {
-      constexpr bool ST = decltype(st_c)::value;
-      constexpr int WAIT = decltype(wait_c)::value;
+    // I/O step `it` (between B(it) and B(it+1)): the loads of tile it+S-1, BM
+    // where it falls, the stores of tile it-2 (J > 0), then the wait for tile
+    // it+1: issued in step it-S+2 (or the prologue), followed by the loads of
+    // S-2 tiles and the stores of the last J steps, S-1 at most -- vector
+    // memory operations of one wave complete in order.
+    auto iostep = [&](int it, auto j_c, auto merge_c) {
+      constexpr int J = decltype(j_c)::value;
       constexpr bool MERGE = decltype(merge_c)::value;
 #pragma unroll
       for (int q = 0; q < BPW; ++q) issue_load(it + S - 1, q);
       if constexpr (MERGE) asm volatile("s_barrier" ::: "memory");
-      if constexpr (ST) store_tile(it - 2);
+      if constexpr (J > 0) store_tile(it - 2);
+      constexpr int WAIT = (S - 2) * BPW + J * SPW;
+      static_assert(J < S && WAIT < 64, "vmcnt");
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(WAIT) : "memory");
     };
     using Y = std::true_type;
     using F = std::false_type;
-    using W8 = std::integral_constant<int, BPW>;
-    using W16 = std::integral_constant<int, BPW + SPW>;
-    using W24 = std::integral_constant<int, BPW + 2 * SPW>;
+    using J0 = std::integral_constant<int, 0>;
 #pragma unroll
     for (int it = 0; it < S - 1; ++it)
 #pragma unroll
       for (int q = 0; q < BPW; ++q) issue_load(it, q);
     wait_loads_barrier<BPW * (S - 1)>();  // BA
     wait_loads_barrier<BPW * (S - 2)>();  // B(0)
-    for (int it = 0; it < nT; ++it) iostep(it, F{}, W8{}, F{});
-    iostep(nT, F{}, W8{}, Y{});
+    for (int it = 0; it < nT; ++it) iostep(it, J0{}, F{});
+    iostep(nT, J0{}, Y{});
     if constexpr (STAGED) {
-      iostep(nT + 1, F{}, W8{}, F{});
-      if (total >= nT + 2) iostep(nT + 2, Y{}, W16{}, F{});  // nT >= 2
-      for (int it = nT + 3; it <= total; ++it) iostep(it, Y{}, W24{}, F{});
+      iostep(nT + 1, J0{}, F{});
+      int it = nT + 2;  // the first step with stores
+      auto ramp = [&](auto j_c) {
+        if (it <= total) iostep(it++, j_c, F{});
+      };
+      if constexpr (S > 2) ramp(std::integral_constant<int, 1>{});
+      if constexpr (S > 3) ramp(std::integral_constant<int, 2>{});
+      if constexpr (S > 4) ramp(std::integral_constant<int, 3>{});
+      if constexpr (S > 5) ramp(std::integral_constant<int, 4>{});
+      static_assert(S <= 6, "ramp");
+      for (; it <= total; ++it) iostep(it, std::integral_constant<int, S - 1>{}, F{});
       // after B(total+1): the last tile's stores
       store_tile(total - 1);
     } else {
-      for (int it = nT + 1; it <= total; ++it) iostep(it, F{}, W8{}, F{});
+      for (int it = nT + 1; it <= total; ++it) iostep(it, J0{}, F{});
     }
     // every direct-to-LDS load has landed before the workgroup's LDS is freed
     // (no barrier: the compute waves have met their last one)
@@ -390,7 +406,7 @@ chain_rows_kernel(const ChainParams p) {
           }
           if constexpr (MMA) {
 #pragma unroll
-            for (int s = 2 * Q; s < 2 * Q + 2; ++s) {
+            for (int s = KPG * Q; s < KPG * (Q + 1); ++s) {
               if constexpr (Q == 0) {
                 if (s == 0) {
                   f32x16 z;
@@ -474,23 +490,23 @@ chain_rows_kernel(const ChainParams p) {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int IN_DT>
+template <int IN_DT, int KS>
 static const void* rows_by_out(int out_dt) {
   switch (out_dt) {
-    case DT_F32: return reinterpret_cast<const void*>(&chain_rows_kernel<IN_DT, DT_F32>);
-    case DT_F16: return reinterpret_cast<const void*>(&chain_rows_kernel<IN_DT, DT_F16>);
-    case DT_BF16: return reinterpret_cast<const void*>(&chain_rows_kernel<IN_DT, DT_BF16>);
+    case DT_F32: return reinterpret_cast<const void*>(&chain_rows_kernel<IN_DT, DT_F32, KS>);
+    case DT_F16: return reinterpret_cast<const void*>(&chain_rows_kernel<IN_DT, DT_F16, KS>);
+    case DT_BF16: return reinterpret_cast<const void*>(&chain_rows_kernel<IN_DT, DT_BF16, KS>);
   }
   return nullptr;
 }
 
-const void* rows_kernel_symbol(int in_dt, int out_dt) {
-  if (in_dt == DT_F16) return rows_by_out<DT_F16>(out_dt);
-  if (in_dt == DT_BF16) return rows_by_out<DT_BF16>(out_dt);
+const void* rows_kernel_symbol(int in_dt, int out_dt, int ksteps) {
+  if (in_dt == DT_F16) return ksteps == 4 ? rows_by_out<DT_F16, 4>(out_dt) : rows_by_out<DT_F16, 8>(out_dt);
+  if (in_dt == DT_BF16) return ksteps == 4 ? rows_by_out<DT_BF16, 4>(out_dt) : rows_by_out<DT_BF16, 8>(out_dt);
   return nullptr;
 }
 
 int rows_kernel_threads() { return rows::NT; }
-int rows_kernel_max_k() { return rows::KS * 16; }
+int rows_kernel_max_k() { return 8 * 16; }
 
 }  // namespace wtc

@@ -58,7 +58,9 @@ const void* wide_kernel_symbol(int in_dt, int out_dt, int epi);
 int wide_kernel_threads();
 
 // One workgroup per 128-row block, two passes over N (K <= rows_kernel_max_k()).
-const void* rows_kernel_symbol(int in_dt, int out_dt);
+// `ksteps`: rows_ksteps of the problem's k.
+const void* rows_kernel_symbol(int in_dt, int out_dt, int ksteps);
+constexpr int rows_ksteps(int64_t k) { return k <= 64 ? 4 : 8; }
 int rows_kernel_threads();
 int rows_kernel_max_k();
 
