@@ -190,12 +190,18 @@ _IN_BYTES = {"f32": 4, "f16": 2, "bf16": 2, "fp8": 1}
 _OUT_BYTES = {"f32": 4, "f16": 2, "bf16": 2}
 # own k-tile cycles per (variant, input class 0 16-bit / 1 fp8 / 2 f32 /
 # 3 f32 on 64 x 64 tiles), fixed cycles per (variant, epilogue 0 exchange /
-# 1 split, class 0 16-bit and fp8 / 2, 3 as above), then scalars
+# 1 split, class 0 16-bit and fp8 / 2, 3 as above; f32's 128 x 128 tiles share
+# one), then scalars
 _KT = [(0, 0), (0, 1), (0, 2), (0, 3), (1, 0), (1, 1), (2, 0), (2, 1), (4, 0), (4, 1)]
-_FX = [(0, 0, 0), (0, 1, 0), (0, 0, 2), (0, 1, 2), (0, 0, 3), (1, 0, 0), (1, 1, 0), (2, 1, 0),
-       (4, 1, 0)]
+_FX = [(0, 0, 0), (0, 1, 0), (0, 1, 2), (0, 0, 3), (1, 0, 0), (1, 1, 0), (2, 1, 0), (4, 1, 0)]
 _SCALARS = ["launch_us", "exchange_us", "exchange_per_tile_us", "hbm_gbs", "feed_gbs",
-            "rows_block_cyc", "rows_tile_cyc", "rows_kstep_cyc"]
+            "rows_block_cyc", "rows_tile_cyc", "rows_tile4_cyc"]
+
+
+# 128-column tiles of more than two waves: what they re-read of A and B
+MANY_WAVES = 1.1
+# a 256 x 256 tile of f32 outputs: its second staging round and store
+WIDE_F32_CYC = 17000.0
 
 
 def _clock_ghz(busy):
@@ -219,7 +225,7 @@ def model_us(x, r, cu=256):
         blocks = b * math.ceil(m / 128)
         waves = math.ceil(blocks / cu)
         f = _clock_ghz(blocks / (waves * cu))
-        cyc = c["rows_block_cyc"] + n_t * (c["rows_tile_cyc"] + c["rows_kstep_cyc"] * math.ceil(k / 16))
+        cyc = c["rows_block_cyc"] + n_t * c["rows_tile4_cyc" if k <= 64 else "rows_tile_cyc"]
         return c["launch_us"] + max(waves * cyc / (f * 1e3), (ab + elems * osz) * us_per_byte)
     rows, cols = _TILE[v]
     cls = 1 if r["in"] == "fp8" else (2 if r["in"] == "f32" else 0)
@@ -229,16 +235,23 @@ def model_us(x, r, cu=256):
         cls = 3
     n_t = math.ceil(n / cols)
     tiles = b * math.ceil(m / rows) * n_t
-    waves = math.ceil(tiles / cu)
-    f = _clock_ghz(tiles / (waves * cu))
     nk = math.ceil(k * isz / 128)
     epi = 0 if r["path"] == "exchange" else 1
     full, rem = tiles // cu, tiles % cu
     t_tiles = 0.0
     for count, active in ((full, cu), (1 if rem else 0, rem)):
         if count:
+            # one full wave and a part of another: each at its own clock; with
+            # more, and with 256 x 256 tiles, at the mean one
+            own = tiles <= 2 * cu and v != 4
+            f = _clock_ghz(active / cu if own else tiles / (math.ceil(tiles / cu) * cu))
             per_kt = kt[(v, cls)] + (rows + cols) * 128 * active * f / c["feed_gbs"]
-            t_tiles += count * (fx[(v, epi, cls if cls >= 2 else 0)] + nk * per_kt) / (f * 1e3)
+            fixed = fx[(v, 1, 2) if cls == 2 else (v, epi, 3 if cls == 3 else 0)]
+            if v == 4 and r["out"] == "f32":
+                fixed += WIDE_F32_CYC
+            t_tiles += count * (fixed + nk * per_kt) / (f * 1e3)
+    if tiles > 2 * cu and v != 4:
+        t_tiles *= MANY_WAVES
     if r["path"] == "exchange":
         t_xch = c["exchange_us"] + c["exchange_per_tile_us"] * n_t if n > cols else 0.0
         return c["launch_us"] + max(t_tiles, (ab + elems * osz) * us_per_byte) + t_xch
@@ -253,8 +266,9 @@ def fit_constants(records):
     from scipy.optimize import least_squares
     recs = [r for r in records if r["path"] != "unfused"]
     x0 = [800.0] * len(_KT) + [5000.0] * len(_FX) + [2.5, 1.0, 0.05, 6000.0, 60000.0, 3000.0,
-                                                      5000.0, 100.0]
-    lo = [0.0] * len(_KT) + [500.0] * len(_FX) + [0.5, 0.0, 0.0, 1000.0, 1000.0, 0.0, 0.0, 0.0]
+                                                      5000.0, 4000.0]
+    # (a row block's A, first tiles and last stores: 1 us at the least)
+    lo = [0.0] * len(_KT) + [500.0] * len(_FX) + [0.5, 0.0, 0.0, 1000.0, 1000.0, 2100.0, 0.0, 0.0]
     res = least_squares(lambda x: np.array([math.log(model_us(x, r) / r["us"]) for r in recs]),
                         np.maximum(x0, np.array(lo) + 1e-6), bounds=(lo, np.inf))
     return res.x

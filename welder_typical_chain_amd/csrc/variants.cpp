@@ -35,7 +35,7 @@ constexpr unsigned kSplitPaths = bit(WTC_PATH_SPLIT) | bit(WTC_PATH_UNFUSED);
 // The constants were fitted (least squares on the log of the time) to
 // back-to-back timings of every variant on every path over the 60 shapes
 // of calibrate.py on MI355X.  Fitted on three of its four shape sets and
-// scored on the fourth, in turn, the fused ranking lost 0.89 % on average
+// scored on the fourth, in turn, the fused ranking lost 0.72 % on average
 // against the measured fastest choice (the hand-written rules it replaces:
 // 5.3 %).
 struct TileCal {
@@ -45,15 +45,15 @@ struct TileCal {
 // [tile variant][0: 16-bit, 1: fp8, 2: f32, 3: f32 64 x 64]; fixed parts shared
 // across 16-bit and fp8 inputs.  Rows: kVarTile128, kVarTile128Loaders, kVarTile256, kVarTile256x256.
 const TileCal kTileCal[4][4] = {
-    /* kVarTile128 */ {{631.76, {3378.7, 5839.9, 0}}, {612.52, {3378.7, 5839.9, 0}}, {2176.7, {4720.4, 6778.6, 0}}, {565.57, {5245.6, 0, 0}}},
-    /* kVarTile128Loaders */ {{558.27, {3771.6, 6373.3, 254}}, {526.47, {3771.6, 6373.3, 254}}, {0, {0, 0, 0}}},
-    /* kVarTile256 */ {{1139.2, {0, 11392.3, 0}}, {1283.0, {0, 11392.3, 0}}, {0, {0, 0, 0}}},
-    /* kVarTile256x256 */ {{1971.5, {0, 20552.0, 6164}}, {1633.1, {0, 20552.0, 6164}}, {0, {0, 0, 0}}},
+    /* kVarTile128 */ {{625.51, {2913.5, 4610.4, 0}}, {627.53, {2913.5, 4610.4, 0}}, {2187.18, {4978.1, 4978.1, 0}}, {593.59, {4509.2, 0, 0}}},
+    /* kVarTile128Loaders */ {{556.60, {3280.5, 5103.1, 254}}, {545.51, {3280.5, 5103.1, 254}}, {0, {0, 0, 0}}},
+    /* kVarTile256 */ {{1159.61, {0, 9359.9, 0}}, {1301.15, {0, 9359.9, 0}}, {0, {0, 0, 0}}},
+    /* kVarTile256x256 */ {{2020.66, {0, 17970.4, 6164}}, {1698.44, {0, 17970.4, 6164}}, {0, {0, 0, 0}}},
 };
 int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
-// Rows kernel, cycles per row block: a fixed part, and per 128-column tile
-// (both passes) a fixed part and a part per 16-wide k-step.
-constexpr double kRowsBlockCyc = 1939.3, kRowsTileCyc = 4930.8, kRowsKstepCyc = 102.65;
+// Rows kernel, cycles per row block: a fixed part, and one per 128-column tile
+// (both passes) with 8 k-steps and with 4 (k <= 64).
+constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4516.7, kRowsTile4Cyc = 3212.1;
 // Few-row kernel: a workgroup's first loads and its softmax (us), one 16 KiB unit
 // of B (us), and the rate at which all workgroups together read B (GB/s): read
 // off 36 timings of 4 to 512 batches x 1 to 16 rows x 256 to 7936 columns (not
@@ -66,13 +66,16 @@ constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFe
 // last tile of a row block: fixed (us) and per column tile (us); the HBM
 // rate of the fused paths' streaming passes and the chip-wide rate that
 // prices k-tile bytes (GB/s).
-constexpr double kLaunchUs = 3.6813, kExchangeUs = 0.3895, kExchangePerTileUs = 0.09190;
-constexpr double kHbmGBs = 7664.6, kFeedGBs = 81910.8;
+constexpr double kLaunchUs = 3.9636, kExchangeUs = 0.3687, kExchangePerTileUs = 0.11020;
+constexpr double kHbmGBs = 6615.1, kFeedGBs = 115179.1;
+// A 256 x 256 tile of f32 outputs takes this much longer (its second staging round
+// and stores; fp8 4 x 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles).
+constexpr double kManyWaves = 1.1, kWideF32Cyc = 17000.0;
 // Unfused row passes (one 256-thread workgroup per row, eight per CU): HBM
 // rate, and the rate one workgroup streams its row at (GB/s).
 constexpr double kRowPassHbmGBs = 5293.0, kRowPassWgGBs = 5.573;
 
-// Core clock under load, from the call's mean share of busy CUs: 1.5 GHz
+// Core clock under load, from the share of busy CUs: 1.5 GHz
 // with every CU busy throughout, ~2.1 with half of them or fewer (the chip's
 // power limit, not the workload, sets it).
 double clock_ghz(double busy) {
@@ -229,7 +232,7 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     }
     const double waves = std::ceil(blocks / cu);
     const double f = clock_ghz(blocks / (waves * cu));
-    const double cyc = kRowsBlockCyc + nT * (kRowsTileCyc + kRowsKstepCyc * (double)cdiv(p.k, 16));
+    const double cyc = kRowsBlockCyc + nT * (p.k <= 64 ? kRowsTile4Cyc : kRowsTileCyc);
     const double t_blocks = waves * cyc / (f * 1e3);
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
     return kLaunchUs + std::max(t_blocks, t_hbm);
@@ -237,16 +240,25 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
   const TileCal& cal = kTileCal[cal_row(v.id)][in_class(p.in_dt) + (ts.rows == 64 ? 1 : 0)];
   const int epi = path == WTC_PATH_EXCHANGE ? 0 : (path == WTC_PATH_SPLIT ? 1 : 2);
   const double tiles = (double)variant_grid(v, path, p);
-  const double waves = std::ceil(tiles / cu);
-  const double f = clock_ghz(tiles / (waves * cu));
   const double nk = (double)cdiv(p.k * in_bytes(p.in_dt), 128);
   const double kt_bytes = (double)(ts.rows + ts.cols) * 128.0;  // A and B per 128 bytes of K
   auto wave_us = [&](double active) {
+    // One full wave and a part of another: each at its own clock (fp8 1000 x 4104
+    // x 2064, 264 tiles of 128 x 128: 35.2 us, where the mean clock gave 26 and
+    // the 256 x 128 tiles take 31.2).  With more waves, whose tiles run side by
+    // side, and with 256 x 256 tiles the mean clock ranked better.
+    const bool own = tiles <= 2 * cu && v.id != kVarTile256x256;
+    const double f = clock_ghz(own ? active / cu : tiles / (std::ceil(tiles / cu) * cu));
     const double kt = cal.kt_cyc + kt_bytes * active * f / kFeedGBs;
-    return (cal.fixed_cyc[epi] + nk * kt) / (f * 1e3);
+    const double wide_f32 = v.id == kVarTile256x256 && epi == 1 && p.out_dt == WTC_DTYPE_F32 ? kWideF32Cyc : 0.0;
+    return (cal.fixed_cyc[epi] + wide_f32 + nk * kt) / (f * 1e3);
   };
   const double full = std::floor(tiles / cu), rem = tiles - full * cu;
-  const double t_tiles = full * wave_us(cu) + (rem > 0 ? wave_us(rem) : 0.0);
+  // 128-column tiles of more than two waves re-read A and B more than the rates
+  // above say: without this part a row of 145 of them was put before 73 tiles of
+  // 256 x 256 (bf16 607 x 18520 x 2240: 101 us, 70 with the latter).
+  const double many = tiles > 2 * cu && v.id != kVarTile256x256 ? kManyWaves : 1.0;
+  const double t_tiles = many * (full * wave_us(cu) + (rem > 0 ? wave_us(rem) : 0.0));
   if (path == WTC_PATH_EXCHANGE) {
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
     const double t_xch = p.n > ts.cols ? kExchangeUs + kExchangePerTileUs * nT : 0.0;
