@@ -71,12 +71,15 @@ extern "C" {
 #define WTC_PATH_AUTO 0      /* the fused path and kernel variant that the library's
                                 cost model (calibrated on MI355X) ranks fastest for
                                 the problem: EXCHANGE, SPLIT or ROWS */
-#define WTC_PATH_EXCHANGE 1  /* one kernel, row statistics exchanged between tiles */
+#define WTC_PATH_EXCHANGE 1  /* one kernel, row statistics exchanged between tiles
+                                that are all resident at once */
 #define WTC_PATH_SPLIT 2     /* two kernels: tile pass + row rescale (online two-pass) */
 #define WTC_PATH_UNFUSED 3   /* five kernels: matmul, max, exp, sum, divide */
 #define WTC_PATH_ROWS 4      /* one kernel, one workgroup per 128 rows over all of n:
                                 row statistics in a first pass, outputs in a second
-                                (16-bit inputs, k <= 128) */
+                                (16-bit inputs, k <= 128); batches of at most 32
+                                rows whose logits fit in LDS: one workgroup and
+                                one pass per batch */
 
 /* The fused chain.  in_dtype is one of F32/F16/BF16/FP8_E4M3; out_dtype one of
  * F32/F16/BF16.  scale_a / scale_b are the per-tensor dequantisation scales

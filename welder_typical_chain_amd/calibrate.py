@@ -202,6 +202,8 @@ _SCALARS = ["launch_us", "exchange_us", "exchange_per_tile_us", "hbm_gbs", "feed
 MANY_WAVES = 1.1
 # a 256 x 256 tile of f32 outputs: its second staging round and store
 WIDE_F32_CYC = 17000.0
+# a 256 x 128 tile's fixed part on the exchange path
+TALL_FIXED_CYC = 11000.0
 
 
 def _clock_ghz(busy):
@@ -233,6 +235,9 @@ def model_us(x, r, cu=256):
             b * math.ceil(m / 64) * math.ceil(n / 64) <= 2 * cu and math.ceil(n / 64) <= 64):
         rows = cols = 64  # tile_shape's rule (csrc/variants.cpp)
         cls = 3
+    tall = v == 1 and r["path"] == "exchange" and b * math.ceil(m / 128) * n_t > cu
+    if tall:
+        rows = 256  # tile_shape's rule, too
     n_t = math.ceil(n / cols)
     tiles = b * math.ceil(m / rows) * n_t
     nk = math.ceil(k * isz / 128)
@@ -245,8 +250,10 @@ def model_us(x, r, cu=256):
             # more, and with 256 x 256 tiles, at the mean one
             own = tiles <= 2 * cu and v != 4
             f = _clock_ghz(active / cu if own else tiles / (math.ceil(tiles / cu) * cu))
-            per_kt = kt[(v, cls)] + (rows + cols) * 128 * active * f / c["feed_gbs"]
+            per_kt = kt[(2 if tall else v, cls)] + (rows + cols) * 128 * active * f / c["feed_gbs"]
             fixed = fx[(v, 1, 2) if cls == 2 else (v, epi, 3 if cls == 3 else 0)]
+            if tall:
+                fixed = TALL_FIXED_CYC
             if v == 4 and r["out"] == "f32":
                 fixed += WIDE_F32_CYC
             t_tiles += count * (fixed + nk * per_kt) / (f * 1e3)

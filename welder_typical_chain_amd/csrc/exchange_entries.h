@@ -11,7 +11,8 @@ namespace wtc {
 // The tiles of a row block (all co-resident) exchange per-row log-sum-exps
 // through tagged entries instead of a barrier.  Tile (row block rbg, column
 // tile nt) owns slot rbg * nT + nt: 128 64-bit entries, one per tile row, at
-// ent + slot * 128.  An entry holds the row's log-sum-exp over the tile's
+// ent + slot * 128 (a 256-row tile owns two: slots 2s and 2s + 1, each with
+// its own generation).  An entry holds the row's log-sum-exp over the tile's
 // columns (f32, log2 domain) in its low word and a tag in its high word, and
 // is written with ONE 64-bit atomic store, so a reader sees either an old
 // entry or the whole new one.  The tag is the slot's generation + 1: every

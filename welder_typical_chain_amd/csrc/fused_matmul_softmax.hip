@@ -7,7 +7,7 @@
 // chain spec mlir/matmul_softmax_chain_f16_native.mlir:7-95).
 //
 // One workgroup owns a TM x 128 output tile (TM = 128; 256 on the split
-// path of large problems).  16-bit and fp8 inputs: 512 threads = 8 waves, 2
+// path of large problems and on the exchange path of middling ones).  16-bit and fp8 inputs: 512 threads = 8 waves, 2
 // per SIMD (the wave layouts are described at Cfg); k-tiles of 128 bytes of
 // K stream through an LDS ring filled by direct-to-LDS buffer loads, B stays
 // K-major in LDS and its MFMA operands are read with LDS transpose reads.  f32
@@ -82,7 +82,8 @@ constexpr int kSlotRows = 128;
 //     SIMD waits to issue a load, the other issues MFMAs); 4 stages of 32 KiB.
 //   LW = 0, TM = 256: a 4x2 grid of 64x64 blocks, 3 stages of 48 KiB (the
 //     split path of large problems: a quarter less L2 and a third less LDS
-//     traffic per MFMA).
+//     traffic per MFMA; the exchange path where 128-row tiles outnumber the
+//     CUs).
 //   LW = 1, TM = 128 (loader waves): 4 MFMA waves, one per SIMD, in a 2x2
 //     grid of 64x64 blocks (a third less LDS read traffic per MFMA than
 //     64x32 blocks), and 4 loader waves that issue every direct-to-LDS load,
@@ -140,13 +141,14 @@ template <int IN_DT, int OUT_DT, int TM = 128, int LW = 0, bool XCH = false> str
   static constexpr int STAGING = TM * PITCH * 4;
   // exchange path: the log-sum-exp table follows the staged tile
   static constexpr int LSE_OFF = (STAGING + 255) / 256 * 256;
-  static constexpr int LSE_END = XCH ? LSE_OFF + 64 * kLsePitch * 4 : STAGING;
+  static constexpr int SLOTS = TM > kSlotRows ? TM / kSlotRows : 1;  // exchange slots per tile
+  static constexpr int LSE_END = XCH && SLOTS == 1 ? LSE_OFF + 64 * kLsePitch * 4 : STAGING;
   static constexpr int RING = Cfg<IN_DT, TM, LW>::kRingBytes;
   static constexpr int UNION = LSE_END > RING ? LSE_END : RING;
   static constexpr int RED_OFF = (UNION + 255) / 256 * 256;
   // wstat[kWavesN][TM] (float2), factor[kWavesN][TM] (float), then the
   // exchange path's tile log-sum-exps [TM] (float) and slot generations [64]
-  static constexpr int TOTAL = RED_OFF + 3 * Cfg<IN_DT, TM, LW>::kWavesN * TM * 4 + TM * 4 + 64 * 4;
+  static constexpr int TOTAL = RED_OFF + 3 * Cfg<IN_DT, TM, LW>::kWavesN * TM * 4 + TM * 4 + SLOTS * 64 * 4;
   static_assert(TOTAL <= 160 * 1024, "LDS");
   // f32 64 x 64 tiles: two workgroups per CU
   static_assert(TM != 64 || TOTAL <= 80 * 1024, "LDS");
@@ -602,7 +604,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
                   uint32_t a_bs32, uint32_t b_bs32, uint32_t grid32, const ChainParams p) {
   using C = Cfg<IN_DT, TM, LW>;
   using L = EpiLayout<IN_DT, OUT_DT, TM, LW, EPI == kEpiExchange>;
-  static_assert(EPI != kEpiExchange || TM <= kSlotRows, "rows of an exchange slot");
+  constexpr int SLOTS = L::SLOTS;  // exchange slots per tile: two for 256 rows
   constexpr int BM = TM;      // tile rows
   constexpr int BN = C::kBN;  // tile columns
   constexpr int NT = C::kThreads;
@@ -648,14 +650,16 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   // 32-bit multiply-adds of the load setup -- which the compiler emits as
   // 64-bit multiply-adds with an undefined high addend that may land on the
   // load's destination register -- the compiler waits for it right there.
-  const uint32_t slot0 = rbg * nT32;
-  uint32_t gen_lane = 0;
+  const uint32_t slot0 = rbg * nT32 * SLOTS;
+  uint32_t gen_lane[SLOTS] = {};
   uint32_t wait_known = 0;  // the longest wait recorded before this launch (record_wait)
   auto load_gen0 = [&]() {
     if constexpr (EPI == kEpiExchange) {
       wait_known = __hip_atomic_load(p.err + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      gen_lane = __hip_atomic_load(p.gen + slot0 + ((uint32_t)lane < nT32 ? (uint32_t)lane : nT32 - 1),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int i = 0; i < SLOTS; ++i)
+        gen_lane[i] = __hip_atomic_load(p.gen + slot0 + ((uint32_t)lane < nT32 ? (uint32_t)lane : nT32 - 1) * SLOTS + i,
+                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   };
 
@@ -1007,11 +1011,14 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   // Exchange path: the generation words of the row block's slots in LDS, and
   // the table of the row block's per-tile log-sum-exps [slot][kLsePitch]
   // (log2 domain; this tile's own slot is filled from its statistics).
-  uint32_t* sgen = reinterpret_cast<uint32_t*>(factor + WN * BM + BM);  // [64]
   float* lse_all = reinterpret_cast<float*>(smem + L::LSE_OFF);
-  const uint32_t own_slot = slot0 + nt;
+  const uint32_t own_slot = slot0 + nt * SLOTS;
+  uint32_t* sgen = reinterpret_cast<uint32_t*>(factor + WN * BM + BM);  // [64 * SLOTS]
   if constexpr (EPI == kEpiExchange)
-    if (t < 64 && (uint32_t)t < nT32) sgen[t] = gen_lane;
+    if (t < 64 && (uint32_t)t < nT32) {
+#pragma unroll
+      for (int i = 0; i < SLOTS; ++i) sgen[t * SLOTS + i] = gen_lane[i];
+    }
   if constexpr (EPI != kEpiLogits) {
     __syncthreads();  // the wave statistics (and slot generations) are in place
     if (t < BM) {
@@ -1019,8 +1026,9 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       if constexpr (EPI == kEpiExchange) {
         // publish the row's log-sum-exp over this tile with this launch's tag
         const float lse = st.x + __builtin_amdgcn_logf(st.y);
-        lse_all[nt * kLsePitch + t] = lse;
-        if (!solo) store_entry(p.ent + (uint64_t)own_slot * kSlotRows + t, lse, sgen[nt] + 1u);
+        if constexpr (SLOTS == 1) lse_all[nt * kLsePitch + t] = lse;
+        if (!solo)
+          store_entry(p.ent + (uint64_t)own_slot * kSlotRows + t, lse, sgen[nt * SLOTS + t / kSlotRows % SLOTS] + 1u);
         // Wait until the entry stores are acknowledged.  Not for ordering --
         // the tags make every entry self-describing -- but measured: without
         // the wait, entries became visible to the other XCDs late on some
@@ -1106,6 +1114,71 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
     if (lane == 0 && !in_time) report_timeout(p.err, p.mailbox);
   };
 
+  // 256-row tiles, whose staged rows leave no LDS for the table: thread h of a
+  // row's P polls the entries of the column tiles q = h, h + P, ... itself (one
+  // wave load is 64 / P consecutive rows of P slots), and merges them into its
+  // running max and sum as below.  kTallMaxColTiles (variants.h) keeps a row to
+  // one group of U loads per thread, in flight together; a second one is a second
+  // round trip between XCDs.  bf16 1500 x 3000 x 1000 (24 tiles a row): this kernel
+  // 24.5 us, the split path's two 20.5 and 7.5.
+  auto poll_row = [&](int r, int h, int P, float* gm, float* gs) {
+    constexpr int U = 16;
+    const int nT = (int)nT32;
+    const float2 st = tile_stat(r);
+    const float own = st.x + __builtin_amdgcn_logf(st.y);
+    bool in_time = true;
+    uint64_t waited = 0;
+    for (int qb = 0; qb < nT; qb += U * P) {
+      uint64_t e[U];
+      bool done[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) done[u] = false;
+      const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+      for (;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int q = qb + u * P + h;
+          // past the last tile, or the own one: some tile's entries, not used
+          if (!done[u] && qb + u * P < nT)
+            e[u] = load_entry(p.ent + (uint64_t)(slot0 + (q < nT ? q : 0) * SLOTS) * kSlotRows + r);
+        }
+        bool all = true;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int q = qb + u * P + h;
+          if (!done[u] && qb + u * P < nT) {
+            const bool none = q >= nT || q == (int)nt;
+            if (__all(none || entry_tag(e[u]) == sgen[(none ? 0 : q) * SLOTS + r / kSlotRows % SLOTS] + 1u) || !in_time)
+              done[u] = true;
+            else
+              all = false;
+          }
+        }
+        if (all) break;
+        __builtin_amdgcn_s_sleep(1);
+        const uint64_t w = __builtin_amdgcn_s_memrealtime() - t0;
+        waited = w > waited ? w : waited;
+        if (w > p.spin_ticks) in_time = false;  // one more pass takes what is there
+      }
+      float nm = *gm;
+      float l[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = qb + u * P + h;
+        l[u] = q >= nT ? -INFINITY : (q == (int)nt ? own : entry_lse(e[u]));
+        nm = fmaxf(nm, l[u]);
+      }
+      const float ref = nm == -INFINITY ? 0.0f : nm;  // no entry at all in this share
+      float cs = *gm == -INFINITY ? 0.0f : *gs * __builtin_amdgcn_exp2f(*gm - ref);
+#pragma unroll
+      for (int u = 0; u < U; ++u) cs += __builtin_amdgcn_exp2f(l[u] - ref);
+      *gm = nm;
+      *gs = cs;
+    }
+    if (lane == 0 && waited > wait_known) record_wait(p.err, waited);
+    if (lane == 0 && !in_time) report_timeout(p.err, p.mailbox);
+  };
+
   if constexpr (EPI == kEpiExchange && LDW) {
     // Loader waves poll as soon as this tile's entries are acknowledged,
     // while the MFMA waves stage the tile.
@@ -1127,7 +1200,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
     if constexpr (EPI == kEpiExchange) {
       __syncthreads();  // the entries are acknowledged, the own log-sum-exps in the table
       stamp(5);
-      if (!solo) {
+      if (SLOTS == 1 && !solo) {
         stamp(13);
         poll_table(wave, NT / 64);
         stamp(14);
@@ -1152,6 +1225,8 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
           gm = ts.x;
           gs = ts.y;
         }
+      } else if constexpr (SLOTS > 1) {
+        poll_row(r, h, P, &gm, &gs);
       } else {
         // Thread h of the row's P merges the tile log-sum-exps q = h, h + P,
         // h + 2P, ... in groups of four: every read is unconditional (an index
@@ -1208,8 +1283,8 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   // Every thread has its entries of the other slots: the next launch's
   // entries of this tile's slot may carry the next tag.
   if constexpr (EPI == kEpiExchange)
-    if (t == 0 && !solo)
-      __hip_atomic_store(p.gen + own_slot, sgen[nt] + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t < SLOTS && !solo)
+      __hip_atomic_store(p.gen + own_slot + t, sgen[nt * SLOTS + t] + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   stamp(9);
 
   // ---- scale, convert and store: 16 output bytes per thread per step -------
@@ -1412,12 +1487,13 @@ static const void* loaders_by_in(int in_dt, int out_dt) {
   return nullptr;
 }
 
-// 256-row tiles: the split path with 16-bit or fp8 inputs.
-static const void* split256_by_in(int in_dt, int out_dt) {
+// 256-row tiles: the split and exchange paths with 16-bit or fp8 inputs.
+template <int EPI>
+static const void* tall_by_in(int in_dt, int out_dt) {
   switch (in_dt) {
-    case DT_F16: return by_out<DT_F16, kEpiSplit, 256, 0>(out_dt);
-    case DT_BF16: return by_out<DT_BF16, kEpiSplit, 256, 0>(out_dt);
-    case DT_FP8: return by_out<DT_FP8, kEpiSplit, 256, 0>(out_dt);
+    case DT_F16: return by_out<DT_F16, EPI, 256, 0>(out_dt);
+    case DT_BF16: return by_out<DT_BF16, EPI, 256, 0>(out_dt);
+    case DT_FP8: return by_out<DT_FP8, EPI, 256, 0>(out_dt);
   }
   return nullptr;
 }
@@ -1440,7 +1516,8 @@ static const void* logits_by_in(int in_dt) {
 const void* chain_kernel_symbol(int in_dt, int out_dt, int epi, int tile_rows, int loaders) {
   if (tile_rows == 256) {
     if (loaders) return nullptr;
-    if (epi == kEpiSplit) return split256_by_in(in_dt, out_dt);
+    if (epi == kEpiExchange) return tall_by_in<kEpiExchange>(in_dt, out_dt);
+    if (epi == kEpiSplit) return tall_by_in<kEpiSplit>(in_dt, out_dt);
     if (epi == kEpiLogits) return out_dt == DT_F32 ? logits_by_in<256, 0>(in_dt) : nullptr;
     return nullptr;
   }
@@ -1492,6 +1569,14 @@ int chain_kernel_lds_bytes(int in_dt, int out_dt, int tile_rows, int loaders) {
   if (in_dt == DT_F32) {
     if (tile_rows == 64) return loaders ? lds_bytes_for<DT_F32, 64, 1>(out_dt) : lds_bytes_for<DT_F32, 64, 0>(out_dt);
     return lds_bytes_for<DT_F32, 128, 1>(out_dt);
+  }
+  if (tile_rows == 256) {
+    switch (in_dt) {
+      case DT_F16: return lds_bytes_for<DT_F16, 256, 0>(out_dt);
+      case DT_BF16: return lds_bytes_for<DT_BF16, 256, 0>(out_dt);
+      case DT_FP8: return lds_bytes_for<DT_FP8, 256, 0>(out_dt);
+    }
+    return 0;
   }
   if (loaders) {
     switch (in_dt) {

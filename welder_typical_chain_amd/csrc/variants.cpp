@@ -35,7 +35,7 @@ constexpr unsigned kSplitPaths = bit(WTC_PATH_SPLIT) | bit(WTC_PATH_UNFUSED);
 // The constants were fitted (least squares on the log of the time) to
 // back-to-back timings of every variant on every path over the 60 shapes
 // of calibrate.py on MI355X.  Fitted on three of its four shape sets and
-// scored on the fourth, in turn, the fused ranking lost 0.72 % on average
+// scored on the fourth, in turn, the fused ranking lost 0.83 % on average
 // against the measured fastest choice (the hand-written rules it replaces:
 // 5.3 %).
 struct TileCal {
@@ -71,6 +71,10 @@ constexpr double kHbmGBs = 6615.1, kFeedGBs = 115179.1;
 // A 256 x 256 tile of f32 outputs takes this much longer (its second staging round
 // and stores; fp8 4 x 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles).
 constexpr double kManyWaves = 1.1, kWideF32Cyc = 17000.0;
+// A 256 x 128 tile's fixed part on the exchange path (its k-tiles cost what the split
+// path's do): read off three timings (modelled and measured us: 1536 x 4096 x 1024
+// bf16 25.6, 24.8; 2560 x 2560 x 1024 f16 24.7, 23.9; 2 x 1536 x 1536 x 512 16.2, 16.5).
+constexpr double kTallFixedCyc = 11000.0;
 // Unfused row passes (one 256-thread workgroup per row, eight per CU): HBM
 // rate, and the rate one workgroup streams its row at (GB/s).
 constexpr double kRowPassHbmGBs = 5293.0, kRowPassWgGBs = 5.573;
@@ -137,14 +141,24 @@ bool variant_by_id(int in_dt, int id, VariantDesc* out) {
   return false;
 }
 
+// Whether tile_shape's 256-row tiles carry the exchange path: 128-row tiles do
+// not fit on the CUs, 256-row tiles do.
+static bool tall_exchange(const VariantDesc& v, const Problem& p) {
+  if (v.id != kVarTile128Loaders) return false;
+  const int64_t nT = cdiv(p.n, 128), tiles = p.batch * cdiv(p.m, 256) * nT;
+  return p.batch * cdiv(p.m, 128) * nT > (int64_t)p.cu_count * std::max(1, p.xch_per_cu) && tiles < p.cu_count &&
+         nT <= kTallMaxColTiles && 2 * tiles <= kExchangeMaxTiles;
+}
+
 bool feasible(const VariantDesc& v, int path, const Problem& p) {
   if (path < WTC_PATH_EXCHANGE || path > WTC_PATH_ROWS || !(v.paths & bit(path))) return false;
   const int64_t nT = cdiv(p.n, v.tile_n);
   switch (path) {
     case WTC_PATH_EXCHANGE: {
       const int64_t tiles = p.batch * cdiv(p.m, v.tile_rows) * nT;
-      return tiles <= (int64_t)p.cu_count * std::max(1, p.xch_per_cu) &&
-             nT <= kExchangeMaxColTiles && tiles <= kExchangeMaxTiles;
+      return (tiles <= (int64_t)p.cu_count * std::max(1, p.xch_per_cu) &&
+              nT <= kExchangeMaxColTiles && tiles <= kExchangeMaxTiles) ||
+             tall_exchange(v, p);
     }
     case WTC_PATH_SPLIT:
       return nT <= kSplitMaxColTiles;
@@ -161,6 +175,7 @@ TileShape tile_shape(const VariantDesc& v, int path, const Problem& p) {
     if (p.m > kFewRows || logits > kFewRowsLogits) return {128, 128, 0, 1};
     return {(int)kFewRows, 128, 0, logits <= kFewRowsLogitsPair && p.batch > p.cu_count ? 2 : 1};
   }
+  if (path == WTC_PATH_EXCHANGE && tall_exchange(v, p)) return {256, 128, 0, 1};
   if (p.in_dt != WTC_DTYPE_F32)
     return {v.tile_rows, (int)v.tile_n, v.loaders, path == WTC_PATH_EXCHANGE ? std::max(1, p.xch_per_cu) : 1};
   if (path == WTC_PATH_EXCHANGE) {
@@ -237,7 +252,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
     return kLaunchUs + std::max(t_blocks, t_hbm);
   }
-  const TileCal& cal = kTileCal[cal_row(v.id)][in_class(p.in_dt) + (ts.rows == 64 ? 1 : 0)];
+  const bool tall = path == WTC_PATH_EXCHANGE && ts.rows == 256;
+  const TileCal& cal = kTileCal[tall ? 2 : cal_row(v.id)][in_class(p.in_dt) + (ts.rows == 64 ? 1 : 0)];
   const int epi = path == WTC_PATH_EXCHANGE ? 0 : (path == WTC_PATH_SPLIT ? 1 : 2);
   const double tiles = (double)variant_grid(v, path, p);
   const double nk = (double)cdiv(p.k * in_bytes(p.in_dt), 128);
@@ -251,7 +267,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     const double f = clock_ghz(own ? active / cu : tiles / (std::ceil(tiles / cu) * cu));
     const double kt = cal.kt_cyc + kt_bytes * active * f / kFeedGBs;
     const double wide_f32 = v.id == kVarTile256x256 && epi == 1 && p.out_dt == WTC_DTYPE_F32 ? kWideF32Cyc : 0.0;
-    return (cal.fixed_cyc[epi] + wide_f32 + nk * kt) / (f * 1e3);
+    const double fixed = tall ? kTallFixedCyc : cal.fixed_cyc[epi];
+    return (fixed + wide_f32 + nk * kt) / (f * 1e3);
   };
   const double full = std::floor(tiles / cu), rem = tiles - full * cu;
   // 128-column tiles of more than two waves re-read A and B more than the rates

@@ -77,6 +77,16 @@ struct TileShape {
 // Short K (up to kF32OneGroupK): one k-group, whose sums need not meet.
 constexpr int kF32SmallTilesPerCu = 2;
 constexpr int64_t kF32OneGroupK = 192;
+// And 16-bit or fp8 inputs on the exchange path when 128-row tiles outnumber the
+// CUs and 256-row tiles (the loader-wave variant's request, run without loader
+// waves) do not.  They leave CUs idle, as they do on the split path, but need no
+// second pass over the output (us, split and exchange: 1500 x 3000 x 1000 bf16
+// 27.7, 24.5; 3328 x 2048 x 512 f16 25.2, 17.4; 15 x 130 x 2048 x 256 bf16 -> f32
+// 23.9, 15.2; 2304 x 2048 x 1024 fp8 23.9, 18.5).  Rows of more than 32 column
+// tiles stay on the split path: a thread would poll a second group of entries
+// (1000 x 4104 x 2064 fp8, 33 tiles: split 31.3, exchange 34.0); and so does a
+// grid that takes every CU, whose plan is pinned (4096 x 2048 x 128, split).
+constexpr int64_t kTallMaxColTiles = 32;
 // And on the rows path: one 32-row block per batch (chain_few_rows_kernel, which
 // reads B once) when the problem has at most that many rows and their logits fit
 // in LDS, kFewRowsLogits floats with each row's columns padded to 128 + 4; two
