@@ -200,8 +200,11 @@ _SCALARS = ["launch_us", "exchange_us", "exchange_per_tile_us", "hbm_gbs", "feed
 
 # 128-column tiles of more than two waves: what they re-read of A and B
 MANY_WAVES = 1.1
-# a 256 x 256 tile of f32 outputs: its second staging round and store
+# a 256 x 256 tile of f32 outputs: its second staging round and store, with
+# fewer than eight k-tiles
 WIDE_F32_CYC = 17000.0
+# a row block's column tile of f32 outputs, all 128 rows stored
+ROWS_TILE_F32_CYC = 1700.0
 # a 256 x 128 tile's fixed part on the exchange path
 TALL_FIXED_CYC = 11000.0
 
@@ -227,7 +230,8 @@ def model_us(x, r, cu=256):
         blocks = b * math.ceil(m / 128)
         waves = math.ceil(blocks / cu)
         f = _clock_ghz(blocks / (waves * cu))
-        cyc = c["rows_block_cyc"] + n_t * c["rows_tile4_cyc" if k <= 64 else "rows_tile_cyc"]
+        cyc = c["rows_block_cyc"] + n_t * (c["rows_tile4_cyc" if k <= 64 else "rows_tile_cyc"] +
+                                        (ROWS_TILE_F32_CYC * min(m, 128) / 128 if osz == 4 else 0.0))
         return c["launch_us"] + max(waves * cyc / (f * 1e3), (ab + elems * osz) * us_per_byte)
     rows, cols = _TILE[v]
     cls = 1 if r["in"] == "fp8" else (2 if r["in"] == "f32" else 0)
@@ -254,7 +258,7 @@ def model_us(x, r, cu=256):
             fixed = fx[(v, 1, 2) if cls == 2 else (v, epi, 3 if cls == 3 else 0)]
             if tall:
                 fixed = TALL_FIXED_CYC
-            if v == 4 and r["out"] == "f32":
+            if v == 4 and r["out"] == "f32" and nk < 8:
                 fixed += WIDE_F32_CYC
             t_tiles += count * (fixed + nk * per_kt) / (f * 1e3)
     if tiles > 2 * cu and v != 4:

@@ -52,16 +52,21 @@ const TileCal kTileCal[4][4] = {
 };
 int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // Rows kernel, cycles per row block: a fixed part, and one per 128-column tile
-// (both passes) with 8 k-steps and with 4 (k <= 64).
-constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4516.7, kRowsTile4Cyc = 3212.1;
+// (both passes) with 8 k-steps and with 4 (k <= 64), and what the stores of
+// 128 rows of f32 outputs add (14 shapes of 12 to 84 row blocks took 15 to 50 % more
+// than modelled without it: 37 x 152 x 1952 x 128 f16 58.6 us, 43.8 with 256-row
+// tiles; 296 x 4 x 5192 x 96, 4 rows stored, does not: 166, split 236).
+constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4516.7, kRowsTile4Cyc = 3212.1, kRowsTileF32Cyc = 1700.0;
 // Few-row kernel: a workgroup's first loads and its softmax (us), one 16 KiB unit
 // of B (us), and the rate at which all workgroups together read B (GB/s): read
 // off 36 timings of 4 to 512 batches x 1 to 16 rows x 256 to 7936 columns (not
 // in the table above, whose shapes have more rows).  For so few rows the model
-// prices the 128-row tiles up to a quarter too high, so the few-row kernel is
-// priced a quarter too high as well: it then lost nowhere against them (16 x 1 x
-// 2304 x 128: 13.8 us, split 11.7; 32 x 2 x 1312 x 128: 10.5 and 12.1).
-constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFewMargin = 1.25;
+// prices the 128-row tiles up to 30 % too high, so the few-row kernel is priced
+// as much too high: it is then taken where it loses by 3 % at the most (split in
+// place of it: 16 x 1 x 2304 x 128 11.7 us against 13.8, 19 x 1 x 4752 x 64 15.2
+// against 17.7; taken: 32 x 2 x 1312 x 128 10.5 us, split 12.1, and 24 x 2 x 5368 x
+// 64 19.4, 18.8).
+constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFewMargin = 1.3;
 // Back-to-back launch cost of one kernel (us); the row exchange after the
 // last tile of a row block: fixed (us) and per column tile (us); the HBM
 // rate of the fused paths' streaming passes and the chip-wide rate that
@@ -69,8 +74,11 @@ constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFe
 constexpr double kLaunchUs = 3.9636, kExchangeUs = 0.3687, kExchangePerTileUs = 0.11020;
 constexpr double kHbmGBs = 6615.1, kFeedGBs = 115179.1;
 // A 256 x 256 tile of f32 outputs takes this much longer (its second staging round
-// and stores; fp8 4 x 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles).
-constexpr double kManyWaves = 1.1, kWideF32Cyc = 17000.0;
+// and stores; fp8 4 x 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles).  With
+// eight k-tiles or more it is left out: the 128-column tiles then lose as much,
+// unmodelled, to B rows that do not start on a cache line (fp8 524 x 51576 x 6816:
+// 256 x 256 tiles 337 us, 128 x 128 547; f16 638 x 40776 x 2368 189, 274).
+constexpr double kManyWaves = 1.1, kWideF32Cyc = 17000.0, kWideF32KTiles = 8.0;
 // A 256 x 128 tile's fixed part on the exchange path (its k-tiles cost what the split
 // path's do): read off three timings (modelled and measured us: 1536 x 4096 x 1024
 // bf16 25.6, 24.8; 2560 x 2560 x 1024 f16 24.7, 23.9; 2 x 1536 x 1536 x 512 16.2, 16.5).
@@ -247,7 +255,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     }
     const double waves = std::ceil(blocks / cu);
     const double f = clock_ghz(blocks / (waves * cu));
-    const double cyc = kRowsBlockCyc + nT * (p.k <= 64 ? kRowsTile4Cyc : kRowsTileCyc);
+    const double f32_cyc = osz == 4 ? kRowsTileF32Cyc * (double)std::min<int64_t>(p.m, 128) / 128 : 0.0;
+    const double cyc = kRowsBlockCyc + nT * ((p.k <= 64 ? kRowsTile4Cyc : kRowsTileCyc) + f32_cyc);
     const double t_blocks = waves * cyc / (f * 1e3);
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
     return kLaunchUs + std::max(t_blocks, t_hbm);
@@ -266,7 +275,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     const bool own = tiles <= 2 * cu && v.id != kVarTile256x256;
     const double f = clock_ghz(own ? active / cu : tiles / (std::ceil(tiles / cu) * cu));
     const double kt = cal.kt_cyc + kt_bytes * active * f / kFeedGBs;
-    const double wide_f32 = v.id == kVarTile256x256 && epi == 1 && p.out_dt == WTC_DTYPE_F32 ? kWideF32Cyc : 0.0;
+    const bool wide = v.id == kVarTile256x256 && epi == 1 && osz == 4 && nk < kWideF32KTiles;
+    const double wide_f32 = wide ? kWideF32Cyc : 0.0;
     const double fixed = tall ? kTallFixedCyc : cal.fixed_cyc[epi];
     return (fixed + wide_f32 + nk * kt) / (f * 1e3);
   };
