@@ -11,11 +11,12 @@ namespace wtc {
 // The tiles of a row block (all co-resident) exchange per-row log-sum-exps
 // through tagged entries instead of a barrier.  Tile (row block rbg, column
 // tile nt) owns slot rbg * nT + nt: 128 64-bit entries, one per tile row, at
-// ent + slot * 128 (a 256-row tile owns two: slots 2s and 2s + 1, each with
-// its own generation).  An entry holds the row's log-sum-exp over the tile's
-// columns (f32, log2 domain) in its low word and a tag in its high word, and
-// is written with ONE 64-bit atomic store, so a reader sees either an old
-// entry or the whole new one.  The tag is the slot's generation + 1: every
+// ent + slot * 128 (a 256-row tile owns two, slots 2s and 2s + 1, or with f32
+// outputs four, each with its own generation).  An entry holds the row's
+// log-sum-exp over the tile's columns (f32, log2 domain; with four slots the
+// row's max in the first two and its sum in the others) in its low word and a
+// tag in its high word, and is written with ONE 64-bit atomic store, so a reader
+// sees either an old entry or the whole new one.  The tag is the slot's generation + 1: every
 // slot has a generation word gen[slot]; the tiles of a row block read the
 // generation words of all its slots at kernel start, and the owner of a slot
 // increments its word at the end, after reading every other slot of its row
@@ -44,15 +45,15 @@ namespace wtc {
 // out sets bit 0 of err[0], counts in err[2], sets the caller's host-visible
 // mailbox word (if any), and the tile goes on with what it has, so the kernel
 // always drains.
-__device__ inline void store_entry(uint64_t* p, float lse, uint32_t tag) {
-  const uint64_t u = (uint64_t)__builtin_bit_cast(uint32_t, lse) | ((uint64_t)tag << 32);
+__device__ inline void store_entry(uint64_t* p, float value, uint32_t tag) {
+  const uint64_t u = (uint64_t)__builtin_bit_cast(uint32_t, value) | ((uint64_t)tag << 32);
   __hip_atomic_store(p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ inline uint64_t load_entry(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ inline uint32_t entry_tag(uint64_t u) { return (uint32_t)(u >> 32); }
-__device__ inline float entry_lse(uint64_t u) { return __builtin_bit_cast(float, (uint32_t)u); }
+__device__ inline float entry_value(uint64_t u) { return __builtin_bit_cast(float, (uint32_t)u); }
 
 __device__ inline void report_timeout(uint32_t* err, uint32_t* mailbox) {
   __hip_atomic_fetch_or(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -141,7 +141,9 @@ template <int IN_DT, int OUT_DT, int TM = 128, int LW = 0, bool XCH = false> str
   static constexpr int STAGING = TM * PITCH * 4;
   // exchange path: the log-sum-exp table follows the staged tile
   static constexpr int LSE_OFF = (STAGING + 255) / 256 * 256;
-  static constexpr int SLOTS = TM > kSlotRows ? TM / kSlotRows : 1;  // exchange slots per tile
+  static constexpr int HALVES = TM > kSlotRows ? TM / kSlotRows : 1;  // 128-row parts of the tile
+  static constexpr int ENT = TM > kSlotRows ? tall_entries(OUT_DT) : 1;  // exchange entries per row
+  static constexpr int SLOTS = HALVES * ENT;  // exchange slots per tile: entry e of part i in slot e * HALVES + i
   static constexpr int LSE_END = XCH && SLOTS == 1 ? LSE_OFF + 64 * kLsePitch * 4 : STAGING;
   static constexpr int RING = Cfg<IN_DT, TM, LW>::kRingBytes;
   static constexpr int UNION = LSE_END > RING ? LSE_END : RING;
@@ -604,7 +606,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
                   uint32_t a_bs32, uint32_t b_bs32, uint32_t grid32, const ChainParams p) {
   using C = Cfg<IN_DT, TM, LW>;
   using L = EpiLayout<IN_DT, OUT_DT, TM, LW, EPI == kEpiExchange>;
-  constexpr int SLOTS = L::SLOTS;  // exchange slots per tile: two for 256 rows
+  constexpr int SLOTS = L::SLOTS;  // exchange slots per tile: one, for 256 rows two or four
   constexpr int BM = TM;      // tile rows
   constexpr int BN = C::kBN;  // tile columns
   constexpr int NT = C::kThreads;
@@ -1024,11 +1026,16 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
     if (t < BM) {
       const float2 st = tile_stat(t);
       if constexpr (EPI == kEpiExchange) {
-        // publish the row's log-sum-exp over this tile with this launch's tag
-        const float lse = st.x + __builtin_amdgcn_logf(st.y);
-        if constexpr (SLOTS == 1) lse_all[nt * kLsePitch + t] = lse;
-        if (!solo)
-          store_entry(p.ent + (uint64_t)own_slot * kSlotRows + t, lse, sgen[nt * SLOTS + t / kSlotRows % SLOTS] + 1u);
+        // publish the row's log-sum-exp over this tile (two entries a row: its
+        // max and its sum) with this launch's tag
+        const float first = L::ENT == 2 ? st.x : st.x + __builtin_amdgcn_logf(st.y);
+        if constexpr (SLOTS == 1) lse_all[nt * kLsePitch + t] = first;
+        if (!solo) {
+          uint64_t* e = p.ent + (uint64_t)own_slot * kSlotRows + t;
+          const uint32_t* gen = sgen + nt * SLOTS + t / kSlotRows % L::HALVES;
+          store_entry(e, first, gen[0] + 1u);
+          if constexpr (L::ENT == 2) store_entry(e + L::HALVES * kSlotRows, st.y, gen[L::HALVES] + 1u);
+        }
         // Wait until the entry stores are acknowledged.  Not for ordering --
         // the tags make every entry self-describing -- but measured: without
         // the wait, entries became visible to the other XCDs late on some
@@ -1097,7 +1104,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
           if (!done[u]) {
             if (__all(entry_tag(e[u]) == sgen[q] + 1u) || !in_time) {
               done[u] = true;
-              lse_all[q * kLsePitch + (hs & (HS - 1)) * 64 + lane] = entry_lse(e[u]);
+              lse_all[q * kLsePitch + (hs & (HS - 1)) * 64 + lane] = entry_value(e[u]);
             } else {
               all = false;
             }
@@ -1118,18 +1125,22 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   // row's P polls the entries of the column tiles q = h, h + P, ... itself (one
   // wave load is 64 / P consecutive rows of P slots), and merges them into its
   // running max and sum as below.  kTallMaxColTiles (variants.h) keeps a row to
-  // one group of U loads per thread, in flight together; a second one is a second
-  // round trip between XCDs.  bf16 1500 x 3000 x 1000 (24 tiles a row): this kernel
-  // 24.5 us, the split path's two 20.5 and 7.5.
+  // one group of U tiles per thread, whose loads are in flight together; a second
+  // one is a second round trip between XCDs.  bf16 1500 x 3000 x 1000 (24 tiles a
+  // row): this kernel 24.5 us, the split path's two 20.5 and 7.5.
+  // ENT = 2 (f32 outputs): a log-sum-exp in one f32 carries the error of the
+  // logarithm and of its own rounding into every output of the row (f16 1500 x
+  // 3000 x 64, relative 2-norm error of the outputs 2.1e-7; split path 1.5e-7),
+  // so max and sum travel in entries of their own, as the split path keeps them.
   auto poll_row = [&](int r, int h, int P, float* gm, float* gs) {
     constexpr int U = 16;
+    constexpr int ENT = L::ENT;
     const int nT = (int)nT32;
     const float2 st = tile_stat(r);
-    const float own = st.x + __builtin_amdgcn_logf(st.y);
     bool in_time = true;
     uint64_t waited = 0;
     for (int qb = 0; qb < nT; qb += U * P) {
-      uint64_t e[U];
+      uint64_t e[ENT][U];
       bool done[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) done[u] = false;
@@ -1139,8 +1150,11 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         for (int u = 0; u < U; ++u) {
           const int q = qb + u * P + h;
           // past the last tile, or the own one: some tile's entries, not used
-          if (!done[u] && qb + u * P < nT)
-            e[u] = load_entry(p.ent + (uint64_t)(slot0 + (q < nT ? q : 0) * SLOTS) * kSlotRows + r);
+          if (!done[u] && qb + u * P < nT) {
+#pragma unroll
+            for (int i = 0; i < ENT; ++i)
+              e[i][u] = load_entry(p.ent + (uint64_t)(slot0 + (q < nT ? q : 0) * SLOTS + i * L::HALVES) * kSlotRows + r);
+          }
         }
         bool all = true;
 #pragma unroll
@@ -1148,7 +1162,11 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
           const int q = qb + u * P + h;
           if (!done[u] && qb + u * P < nT) {
             const bool none = q >= nT || q == (int)nt;
-            if (__all(none || entry_tag(e[u]) == sgen[(none ? 0 : q) * SLOTS + r / kSlotRows % SLOTS] + 1u) || !in_time)
+            const uint32_t* gen = sgen + (none ? 0 : q) * SLOTS + r / kSlotRows % L::HALVES;
+            bool here = true;
+#pragma unroll
+            for (int i = 0; i < ENT; ++i) here &= entry_tag(e[i][u]) == gen[i * L::HALVES] + 1u;
+            if (__all(none || here) || !in_time)
               done[u] = true;
             else
               all = false;
@@ -1160,20 +1178,30 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         waited = w > waited ? w : waited;
         if (w > p.spin_ticks) in_time = false;  // one more pass takes what is there
       }
+      const float own = ENT == 2 ? st.x : st.x + __builtin_amdgcn_logf(st.y);
       float nm = *gm;
       float l[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int q = qb + u * P + h;
-        l[u] = q >= nT ? -INFINITY : (q == (int)nt ? own : entry_lse(e[u]));
+        l[u] = q >= nT ? -INFINITY : (q == (int)nt ? own : entry_value(e[0][u]));
         nm = fmaxf(nm, l[u]);
       }
       const float ref = nm == -INFINITY ? 0.0f : nm;  // no entry at all in this share
-      float cs = *gm == -INFINITY ? 0.0f : *gs * __builtin_amdgcn_exp2f(*gm - ref);
+      // four partial sums: a quarter of the roundings on the way to each
+      float cs[4] = {*gm == -INFINITY ? 0.0f : *gs * __builtin_amdgcn_exp2f(*gm - ref), 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int u = 0; u < U; ++u) cs += __builtin_amdgcn_exp2f(l[u] - ref);
+      for (int u = 0; u < U; ++u) {
+        const float x = __builtin_amdgcn_exp2f(l[u] - ref);
+        if constexpr (ENT == 2) {
+          const int q = qb + u * P + h;
+          cs[u & 3] += x * (q >= nT ? 0.0f : (q == (int)nt ? st.y : entry_value(e[1][u])));
+        } else {
+          cs[u & 3] += x;
+        }
+      }
       *gm = nm;
-      *gs = cs;
+      *gs = (cs[0] + cs[1]) + (cs[2] + cs[3]);
     }
     if (lane == 0 && waited > wait_known) record_wait(p.err, waited);
     if (lane == 0 && !in_time) report_timeout(p.err, p.mailbox);
@@ -1265,7 +1293,8 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       // thread (r, h < WN) owns the factor of row r, column slice of wave h:
       // exp2(m_w - M) / S.  (Not exp2(m_w - (M + log2 S)): rounding that sum to
       // f32 costs up to 3e-7 of the output once the row is a few hundred wide.)
-      const float inv = __builtin_amdgcn_rcpf(S);
+      // The reciprocal of the hardware, 1 ulp, shows in f32 outputs: a division there.
+      const float inv = L::ENT == 2 ? 1.0f / S : __builtin_amdgcn_rcpf(S);
       if (h < WN) {
         const float mw = wstat[h * BM + r].x;
         factor[h * BM + r] = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw - M) * inv;

@@ -49,6 +49,8 @@ int exchange_lds_pad(int in_dt, int out_dt, const TileShape& ts, int64_t grid, i
 }
 
 static_assert(kExchangeMaxTiles == kMaxExchangeTiles, "exchange slot limit");
+static_assert(tall_slots(DT_F32) == 2 * tall_entries(DT_F32) && tall_slots(DT_F16) == 2 * tall_entries(DT_F16),
+              "slots of a 256-row tile");
 static_assert(kFewRowsLogits == kFewRowsMaxLogits && kFewRowsLogitsPair == kFewRowsPairLogits && kFewRowsPad == 4,
               "few-row kernel limits");
 }  // namespace wtc
@@ -63,7 +65,8 @@ constexpr int kMaxDevices = 64;
 // Timeout mailbox words per device: slot 0 is shared by the streams that
 // found every other slot taken, slots 1.. belong to one stream each.
 constexpr int kMailboxSlots = 64;
-constexpr int64_t kMinDefaultWorkspace = 1 << 20;
+// Holds the entries of any exchange call (kMaxExchangeTiles slots of 1 KiB).
+constexpr int64_t kMinDefaultWorkspace = 2 << 20;
 
 thread_local std::string g_last_error;
 std::atomic<uint64_t> g_spin_ticks{0};  // 0: derived from the plan's estimate
@@ -111,7 +114,7 @@ struct WsLayout {
   int64_t total;
 };
 
-WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int path) {
+WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int out_dt, int path) {
   WsLayout w{};
   const int64_t nT = ceil_div(n, kTile);
   w.gen_off = kGenOff;
@@ -122,6 +125,10 @@ WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int path) {
   if (in_dt == DT_F32) {  // 64 x 64 tiles, when the exchange path runs them: a slot each
     const int64_t tiles = batch * ceil_div(m, 64) * ceil_div(n, 64);
     if (tiles <= kMaxExchangeTiles && tiles * kTile * 8 > exch_bytes) exch_bytes = tiles * kTile * 8;
+  }
+  if (in_dt != DT_F32) {  // 256 x 128 tiles, when the exchange path runs them
+    const int64_t slots = batch * ceil_div(m, 256) * nT * tall_slots(out_dt);
+    if (slots <= kMaxExchangeTiles && slots * kTile * 8 > exch_bytes) exch_bytes = slots * kTile * 8;
   }
   w.stats_bytes = align256(split_bytes > exch_bytes ? split_bytes : exch_bytes);
   w.total = w.stats_off + w.stats_bytes;
@@ -209,7 +216,7 @@ int plan_impl(int64_t batch, int64_t m, int64_t n, int64_t k, int in_dt, int out
   out->path = c.path;
   out->ts = tile_shape(c.v, c.path, pr);
   out->grid = grid;
-  out->ws = ws_layout(batch, m, n, in_dt, c.path).total;
+  out->ws = ws_layout(batch, m, n, in_dt, out_dt, c.path).total;
   out->est_us = c.est_us;
   return WTC_OK;
 }
@@ -747,7 +754,7 @@ int64_t wtc_matmul_softmax_workspace_size(int64_t batch, int64_t m, int64_t n, i
                                           int in_dtype, int out_dtype, int path) {
   g_last_error.clear();
   if (check_args(batch, m, n, k, in_dtype, out_dtype, path)) return -1;
-  return ws_layout(batch, m, n, in_dtype, path).total;
+  return ws_layout(batch, m, n, in_dtype, out_dtype, path).total;
 }
 
 int wtc_workspace_init(void* workspace, size_t workspace_bytes, void* stream) {
@@ -920,7 +927,7 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
     rc = default_workspace(ds, need, &ws, stream);
     if (rc) return rc;
   }
-  const WsLayout L = ws_layout(batch, m, n, in_dtype, chosen);
+  const WsLayout L = ws_layout(batch, m, n, in_dtype, out_dtype, chosen);
   uint8_t* wsb = static_cast<uint8_t*>(ws);
 
   const int isz = dtype_bytes(in_dtype), osz = dtype_bytes(out_dtype);

@@ -34,6 +34,9 @@ enum : int { DT_F32 = 0, DT_F16 = 1, DT_BF16 = 2, DT_FP8 = 3 };
 WTC_HD constexpr int dtype_bytes(int dt) {
   return dt == DT_F32 ? 4 : (dt == DT_FP8 ? 1 : 2);
 }
+// Exchange entries that a row of a 256-row tile publishes: its log-sum-exp, or
+// with f32 outputs its max and its sum.
+WTC_HD constexpr int tall_entries(int out_dt) { return out_dt == DT_F32 ? 2 : 1; }
 
 constexpr int kChunkBytes = 16;
 constexpr int kKTileBytes = 128;

@@ -155,7 +155,7 @@ static bool tall_exchange(const VariantDesc& v, const Problem& p) {
   if (v.id != kVarTile128Loaders) return false;
   const int64_t nT = cdiv(p.n, 128), tiles = p.batch * cdiv(p.m, 256) * nT;
   return p.batch * cdiv(p.m, 128) * nT > (int64_t)p.cu_count * std::max(1, p.xch_per_cu) && tiles < p.cu_count &&
-         nT <= kTallMaxColTiles && 2 * tiles <= kExchangeMaxTiles;
+         nT <= kTallMaxColTiles && tall_slots(p.out_dt) * tiles <= kExchangeMaxTiles;
 }
 
 bool feasible(const VariantDesc& v, int path, const Problem& p) {

@@ -18,6 +18,8 @@
 #include <string>
 #include <vector>
 
+#include "wtc/wtc_hip.h"
+
 namespace wtc {
 
 enum VariantId : int {
@@ -87,6 +89,9 @@ constexpr int64_t kF32OneGroupK = 192;
 // (1000 x 4104 x 2064 fp8, 33 tiles: split 31.3, exchange 34.0); and so does a
 // grid that takes every CU, whose plan is pinned (4096 x 2048 x 128, split).
 constexpr int64_t kTallMaxColTiles = 32;
+// Exchange slots such a tile takes: one per 128 rows and, with f32 outputs, two
+// (the row's max and its sum).
+constexpr int64_t tall_slots(int out_dt) { return out_dt == WTC_DTYPE_F32 ? 4 : 2; }
 // And on the rows path: one 32-row block per batch (chain_few_rows_kernel, which
 // reads B once) when the problem has at most that many rows and their logits fit
 // in LDS, kFewRowsLogits floats with each row's columns padded to 128 + 4; two
