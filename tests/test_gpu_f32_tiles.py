@@ -70,9 +70,11 @@ def test_tile_edges(native_lib, batch, m, n, k):
 @needs_gpu
 @pytest.mark.parametrize("path", ["exchange", "split", "unfused"])
 @pytest.mark.parametrize("m,n,k", [(130, 200, 100), (130, 200, 300)])
-@pytest.mark.parametrize("what", ["tiny", "huge", "zero", "part_subnormal"])
+@pytest.mark.parametrize("what", ["tiny", "huge", "zero", "part_subnormal", "probabilities", "tiny_products"])
 def test_values_past_the_split(native_lib, path, m, n, k, what):
-    """Magnitudes whose bf16 parts would be subnormal or infinite, and zeros."""
+    """Magnitudes whose bf16 parts would be subnormal or infinite, zeros,
+    probabilities (down to 1e-45, recomputed or not the same to f32), and
+    products of ordinary values that are themselves tiny."""
     from welder_typical_chain_amd.chain import matmul_softmax
     print(f"\n[gpu-case] f32 {what} {path} {m}x{n}x{k}", flush=True)
     a, b = _inputs(1, m, n, k, seed=5, spread=2.0)
@@ -86,10 +88,15 @@ def test_values_past_the_split(native_lib, path, m, n, k, what):
         a[0, 7] = 0.0
         b[0, :, 9] = 0.0
         a[0, :, 40:70] = 0.0
+    elif what == "probabilities":
+        a = torch.softmax(a * (30.0 * math.sqrt(k)), dim=-1)
+        assert bool(((a > 0) & (a < 2.0 ** -100)).any())
+    elif what == "tiny_products":
+        a, b = a * 2.0 ** -60, b * 2.0 ** -60
     else:
         a[0, 11, 4] = 1.1754944e-38
         b[0, 5, 66] = 1e-42
-    scale = 4.0 if what == "huge" else 1.0
+    scale = {"huge": 4.0, "tiny_products": 2.0 ** 120}.get(what, 1.0)
     out = matmul_softmax(a[0].cuda(), b[0].cuda(), logit_scale=scale, path=path)
     _check(out[None], a, b, scale)
 
@@ -131,3 +138,31 @@ def test_no_further_from_64_bits_than_f32_products(native_lib, m, n, k):
     err = float((got - want).norm() / want.norm())
     # the kernel's own softmax arithmetic (exp2, sums, product) is in f32 too
     assert err <= 1.5 * float((f32 - want).norm() / want.norm()) + 3e-7, err
+
+
+@needs_gpu
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (2048, 2048, 512)])
+def test_probabilities_take_no_longer(native_lib, m, n, k):
+    """Values below 2^-100 beside ones near 1 do not reach a result: no tile is
+    recomputed for them (that takes 1.5 times the call, and did three times)."""
+    from welder_typical_chain_amd.chain import matmul_softmax
+    print(f"\n[gpu-case] f32 time with tiny values {m}x{n}x{k}", flush=True)
+    a, b = (x[0].cuda() for x in _inputs(1, m, n, k, seed=3))
+    tiny = a.clone()
+    tiny[::17, ::13] = 1e-32
+    out = torch.empty((m, n), device="cuda")
+
+    def us(x):
+        best = math.inf
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            for _ in range(50):
+                matmul_softmax(x, b, out=out)
+            t1.record()
+            torch.cuda.synchronize()
+            best = min(best, t0.elapsed_time(t1) * 20)
+        return best
+    us(a)
+    plain, with_tiny = us(a), us(tiny)
+    assert with_tiny < 1.25 * plain, (with_tiny, plain)

@@ -174,20 +174,33 @@ __device__ inline uint32_t bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
 // error of the outputs, N(0, 1) logits, 1024 x 1024 x 1024: 5.5e-7, with f32
 // MFMAs 1.1e-6).
 //
-// Values that do not split: magnitudes below 2^-100 (a part would be subnormal;
-// the least magnitude of the tile's values tells, Tiny) and infinities, NaN and
-// values that round to an infinite x0 (x - x0 is then NaN or infinite, and so
-// is an accumulator at the end).  The workgroup then recomputes its tile with
-// f32 MFMAs (f32_tile_exactly).
+// Values that do not split: infinities, NaN and values that round to an infinite
+// x0 (x - x0 is then NaN or infinite, and so is an accumulator at the end), and
+// magnitudes below 2^-100, a part of which may be subnormal and read as zero.
+// Such a value loses 2^-125 at most, which matters only beside a large enough
+// value of the other operand and a large enough scale (kTinyMatters).  The
+// accumulators in question are then recomputed with f32 MFMAs (f32_block_exactly):
+// in the first case the wave's 32 x 32 blocks that are not finite, in the second
+// the workgroup's tile.
 // -------------------------------------------------------------------------
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
-// The least nonzero magnitude seen: as 2 * bits - 1, which puts zero last.
-struct Tiny {
+// The least nonzero magnitude seen, as 2 * bits - 1, which puts zero last, and
+// the largest.
+struct Range {
   uint32_t least = 0xFFFFFFFFu;
-  __device__ inline void see(uint32_t x, uint32_t y) { least = min(least, min((x << 1) - 1u, (y << 1) - 1u)); }
-  __device__ inline bool none() const { return least >= (27u << 24) - 1u; }  // 2^-100
+  float most = 0.0f;
+  __device__ inline void see(uint32_t x, uint32_t y) {
+    least = min(least, min((x << 1) - 1u, (y << 1) - 1u));
+    most = fmaxf(fmaxf(most, fabsf(__builtin_bit_cast(float, x))), fabsf(__builtin_bit_cast(float, y)));
+  }
+  __device__ inline bool tiny() const { return least < (27u << 24) - 1u; }  // 2^-100
 };
+// K products, in each of which both values may have lost 2^-125 beside one of
+// magnitude `most`, move a logit (log2 units: c2 times the sum) by at most
+// |c2| K 2^-124 most: 2^-36, a 4096th of an output's f32 rounding, while most is
+// below this over |c2| K.  Probabilities (2^-100 and less beside 1) stay below it.
+constexpr float kTinyMatters = 0x1p88f;
 
 // The three parts of the pair (x, y), each two packed bf16.
 __device__ inline u32x3 split_pair(uint32_t xb, uint32_t yb) {
@@ -258,19 +271,19 @@ template <int TM, int NT> struct F32Regs {
     for (int i = 0; i < V; ++i) b[i] = bload16(w.rb, off + (ok ? 16u * i : 0u));
   }
   // Splits the values and writes their parts to the planes of a stage.
-  __device__ inline void store(uint8_t* stage, int t, Tiny& tiny) const {
+  __device__ inline void store(uint8_t* stage, int t, Range& seen) const {
     const int row = t / TPA, ak = (t % TPA) * E, bk = t / TPB, bn = (t % TPB) * E;
-    put(a, stage + a64_lds_offset(row, ak >> 3) + (ak & 7) * 2, Cfg<DT_F32, TM>::kAPlane, tiny);
-    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_offset<TM>(bk, bn), Cfg<DT_F32, TM>::kBPlane, tiny);
+    put(a, stage + a64_lds_offset(row, ak >> 3) + (ak & 7) * 2, Cfg<DT_F32, TM>::kAPlane, seen);
+    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_offset<TM>(bk, bn), Cfg<DT_F32, TM>::kBPlane, seen);
   }
-  static __device__ inline void put(const u32x4 (&v)[V], uint8_t* dst, int plane, Tiny& tiny) {
+  static __device__ inline void put(const u32x4 (&v)[V], uint8_t* dst, int plane, Range& seen) {
     u32x3 w[2 * V];
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       const u32x4 x = v[i];
-      tiny.see(x[0], x[1]);
+      seen.see(x[0], x[1]);
       w[2 * i] = split_pair(x[0], x[1]);
-      tiny.see(x[2], x[3]);
+      seen.see(x[2], x[3]);
       w[2 * i + 1] = split_pair(x[2], x[3]);
     }
 #pragma unroll
@@ -326,40 +339,58 @@ template <int TM, int MT, int NTN, int KS> struct F32Frags {
   }
 };
 
-// The wave's block with f32 MFMAs, operands straight from memory: for tiles
-// with values that do not split.  k-group g of `groups` takes every
-// `groups`-th pair of k.
-template <int MT, int NTN>
-__device__ inline void f32_tile_exactly(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, uint32_t row,
-                                        uint32_t col, uint32_t M, uint32_t N, uint32_t K, uint32_t lda,
-                                        uint32_t ldb, int lane, int g, int groups, f32x16 (&acc)[MT][NTN]) {
+// A block of 32 x 32 with f32 MFMAs, operands straight from memory: for values
+// that do not split.  With two k-groups group g takes the k it has in the main
+// loop, 16g .. 16g + 15 of each 32 (the other group may keep its sums).  32 k at
+// a time, 16 per lane half, of which MFMA e takes the e-th of both halves; the
+// next 32 are in flight under the MFMAs.  Measured with one infinity in B (us a
+// call; f32 MFMAs throughout 79, 28.5; a round trip to L2 for every 2 k 80, 52):
+// 1024 x 1024 x 1024 37, 512 x 4096 x 256 30.
+template <int GROUPS> struct ExactFrags {
+  static constexpr uint32_t STEP = 32u * GROUPS;           // k from one set to the next
+  static constexpr uint32_t GAP = GROUPS == 2 ? 32u : 8u;  // from a lane's first 8 k to its second
+  u32x4 a[4];
+  uint32_t b[16];
+  // row and col: the lane's; k: its first
+  __device__ inline void load(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, uint32_t row, uint32_t col,
+                              uint32_t k, uint32_t M, uint32_t N, uint32_t K, uint32_t lda, uint32_t ldb) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NTN; ++nt)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.0f;
-  for (uint32_t kp = 2u * (uint32_t)g; kp < K; kp += 2u * (uint32_t)groups) {
-    const uint32_t k = kp + (uint32_t)(lane >> 5);
-    float a[MT], b[NTN];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const uint32_t r = row + (uint32_t)(mt * 32 + (lane & 31));
-      const uint32_t x = bload4(ra, r < M && k < K ? r * lda + k * 4u : kOutOfRange);
-      a[mt] = __builtin_bit_cast(float, x);
+    for (int i = 0; i < 4; ++i) {  // K is a multiple of 4
+      const uint32_t ka = k + 4u * (i & 1) + GAP * (i >> 1);
+      a[i] = bload16(ra, row < M && ka < K ? row * lda + ka * 4u : kOutOfRange);
     }
 #pragma unroll
-    for (int nt = 0; nt < NTN; ++nt) {
-      const uint32_t n = col + (uint32_t)(nt * 32 + (lane & 31));
-      const uint32_t x = bload4(rb, n < N && k < K ? k * ldb + n * 4u : kOutOfRange);
-      b[nt] = __builtin_bit_cast(float, x);
+    for (int e = 0; e < 16; ++e) {
+      const uint32_t kb = k + (uint32_t)(e & 7) + GAP * (uint32_t)(e >> 3);
+      b[e] = bload4(rb, col < N && kb < K ? kb * ldb + col * 4u : kOutOfRange);
     }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < NTN; ++nt)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[nt], a[mt], acc[mt][nt], 0, 0, 0);
   }
+};
+template <int GROUPS>
+__device__ __forceinline__ f32x16 f32_block_exactly(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb,
+                                                    uint32_t row, uint32_t col, uint32_t M, uint32_t N, uint32_t K,
+                                                    uint32_t lda, uint32_t ldb, int lane, int g) {
+  f32x16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  row += (uint32_t)(lane & 31);
+  col += (uint32_t)(lane & 31);
+  uint32_t k = (GROUPS == 2 ? 16u * (uint32_t)g + 8u * (uint32_t)(lane >> 5) : 16u * (uint32_t)(lane >> 5));
+  ExactFrags<GROUPS> cur, next;
+  cur.load(ra, rb, row, col, k, M, N, K, lda, ldb);
+  for (uint32_t kc = 0; kc < K; kc += ExactFrags<GROUPS>::STEP) {  // uniform: lanes past K add zeros
+    k += ExactFrags<GROUPS>::STEP;
+    next.load(ra, rb, row, col, k, M, N, K, lda, ldb);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const u32x4 a4 = cur.a[e / 4];
+      const uint32_t aw = a4[e % 4], bw = cur.b[e];
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, bw), __builtin_bit_cast(float, aw), acc,
+                                                 0, 0, 0);
+    }
+    cur = next;
+  }
+  return acc;
 }
 
 // -------------------------------------------------------------------------
@@ -808,14 +839,18 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
     const uint8_t* b_b = b_in + (uint64_t)bt * b_bs32;
     const typename Regs::Where w =
         Regs::where(a_b, b_b, a_bs32, b_bs32, (uint32_t)row0, (uint32_t)n0, M32, N32, K32, lda32, ldb32, t);
-    uint32_t* redo = reinterpret_cast<uint32_t*>(smem + L::RED_OFF);  // a value of the tile does not split
-    if (t == 0) *redo = 0u;
-    Tiny tiny;
+    // some value of the tile: is tiny; is large enough for a tiny one to matter
+    uint32_t* redo = reinterpret_cast<uint32_t*>(smem + L::RED_OFF);
+    if (t < 2) redo[t] = 0u;
+    Range seen;
     Regs R[PF];
 #pragma unroll
     for (int q = 0; q < PF; ++q) R[q].load(w, q);
+    // read here, under the first loads: the parameter block comes from memory
+    float reach = fabsf(p.c2) * (float)K32;
+    asm volatile("" : "+v"(reach));
     auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    R[0].store(smem, t, tiny);
+    R[0].store(smem, t, seen);
     R[0].load(w, PF);
     meet();
     auto iteration = [&](auto q_c, int kt) {
@@ -823,7 +858,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       Frags F;
       F.read(smem + (kt & 1) * STAGE, lane, wm, nw, kg);
       F.products(acc);
-      R[(Q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE, t, tiny);
+      R[(Q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE, t, seen);
       R[(Q + 1) % PF].load(w, kt + 1 + PF);
       // The scheduler's order: the fragment reads, then the splitting spread
       // over the MFMAs.  In source order a wave would first issue its MFMAs,
@@ -850,18 +885,35 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         if (++kt == nk) break;
       }
     }
-    bool fine = tiny.none();
+    if (seen.tiny()) redo[0] = 1u;
+    if (seen.most * reach > kTinyMatters) redo[1] = 1u;
+    uint32_t blocks = 0;  // the wave's blocks to recompute, bit mt * NTN + j
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int j = 0; j < NTN; ++j)
+      for (int j = 0; j < NTN; ++j) {
+        bool fine = true;
 #pragma unroll
         for (int v = 0; v < 16; ++v) fine &= __builtin_isfinite(acc[mt][j][v]);
-    if (!fine) *redo = 1u;
+        blocks |= __all(fine) ? 0u : 1u << (mt * NTN + j);
+      }
     meet();
-    if (*redo)
-      f32_tile_exactly<MT, NTN>(w.ra, w.rb, (uint32_t)row0 + (uint32_t)(wm * WM), (uint32_t)(n0 + nw), M32, N32,
-                                K32, lda32, ldb32, lane, kg, GROUPS, acc);
+    if (redo[0] & redo[1]) blocks = (1u << (MT * NTN)) - 1u;
+    blocks = __builtin_amdgcn_readfirstlane(blocks);
+    if (__builtin_expect(blocks != 0u, 0)) {
+#pragma unroll 1
+      for (int i = 0; i < MT * NTN; ++i) {
+        if (!(blocks >> i & 1u)) continue;
+        const f32x16 x = f32_block_exactly<GROUPS>(
+            w.ra, w.rb, (uint32_t)row0 + (uint32_t)(wm * WM + i / NTN * 32), (uint32_t)(n0 + nw + i % NTN * 32),
+            M32, N32, K32, lda32, ldb32, lane, kg);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int j = 0; j < NTN; ++j)
+            if (i == mt * NTN + j) acc[mt][j] = x;
+      }
+    }
     if constexpr (GROUPS == 2) {
       // the groups' sums meet through the ring, 16 bytes per lane per step
       f32x4* mrg = reinterpret_cast<f32x4*>(smem) + (wave % C::kMfmaWaves) * (MT * NTN * 4 * 64) + lane;
