@@ -1,10 +1,12 @@
 """CPU checks of the f32 tiles: the LDS layout of a 64-column bf16 plane
-(f32_btr64_offset) and the rule that picks the 64 x 64 tiles (tile_shape)."""
+(f32_btr64_offset), the rule that picks the 64 x 64 tiles (tile_shape), and
+the bound of the partial products that the bf16 split leaves out."""
 from __future__ import annotations
 
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 from welder_typical_chain_amd import _lib
@@ -65,3 +67,30 @@ def test_tile_rule(native_lib, batch, m, n, k, path, grid):
     # every tile of the exchange path has its slot in the workspace
     if path == _lib.PATH_EXCHANGE:
         assert pl["workspace_bytes"] >= 256 + 4096 + grid * 1024
+
+
+def _bf16(x):
+    """x (f32) rounded to bf16, to nearest even, as f32."""
+    u = x.view(np.uint32)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(np.float32)
+
+
+def test_bound_of_the_products_left_out():
+    """Over every mantissa: x0 + x1 + x2 is x, and a1 b2 + a2 b1 + a2 b2 of any two
+    values is at most 2^-24 + 2^-34 of their product, nearly reached; over random
+    pairs its mean square is below 2^-27 and its sign even."""
+    x = (np.arange(2 ** 23, dtype=np.uint32) | 0x3F800000).view(np.float32)
+    x0 = _bf16(x)
+    x1 = _bf16(x - x0)
+    x2 = x - x0 - x1
+    assert np.array_equal(_bf16(x2), x2)
+    assert np.array_equal(x0.astype(np.float64) + x1 + x2, x.astype(np.float64))
+    r1, r2 = x1.astype(np.float64) / x, x2.astype(np.float64) / x
+    most1, most2 = np.abs(r1).max(), np.abs(r2).max()
+    assert 2 * most1 * most2 + most2 ** 2 <= 2.0 ** -24 + 2.0 ** -34
+    worst = np.abs(2 * r1 * r2 + r2 * r2)
+    assert worst.max() > 2.0 ** -24.02 and abs(float(x[worst.argmax()]) - 1.0039) < 1e-4
+    rng = np.random.default_rng(1)
+    i, j = (rng.integers(0, x.size, 1_000_000) for _ in range(2))
+    out = r1[i] * r2[j] + r2[i] * r1[j] + r2[i] * r2[j]
+    assert np.sqrt(np.mean(out ** 2)) < 2.0 ** -27 and abs(out.mean()) < 2.0 ** -35

@@ -4,7 +4,7 @@ parts, and that it is no further from 64 bits than a f32 product.
 
 Tolerance: each of the (at most K + 8) f32 roundings of a logit's sum is at
 most 2^-24 of the sum of its magnitudes S = scale * sum |a b|, the partial
-products left out 2^-26 of it; the softmax turns a logit error d into a
+products left out 2^-24 of it (test_f32_layout.py); the softmax turns a logit error d into a
 relative one of at most 2 d (its own and the row sum's), to which exp2, the
 row sum (N / 128 partial sums) and the final product add a few 2^-22.
 """
@@ -166,3 +166,28 @@ def test_probabilities_take_no_longer(native_lib, m, n, k):
     us(a)
     plain, with_tiny = us(a), us(tiny)
     assert with_tiny < 1.25 * plain, (with_tiny, plain)
+
+
+@needs_gpu
+@pytest.mark.parametrize("m,n,k", [(256, 512, 64), (512, 512, 1024), (1500, 2000, 256)])
+def test_mantissas_at_the_worst_of_the_split(native_lib, m, n, k):
+    """All products of one sign, both operands within 3 units in the last place of
+    1 + 2^-8 - 2^-17, where the partial products left out are 2^-24 of each
+    product: they add up to S 2^-24 per logit (S = 8 here).  Allowed beside it: the
+    roundings of a sum that grows to S in t = 6 K / 16 steps, of either sign and
+    evenly spread over half a unit (0.29 sqrt(t / 3) of 2^-24 S in the mean
+    square), both doubled by the softmax, and its own arithmetic (exp2, sums,
+    product)."""
+    from welder_typical_chain_amd.chain import matmul_softmax
+    print(f"\n[gpu-case] f32 worst mantissas {m}x{n}x{k}", flush=True)
+    g = torch.Generator().manual_seed(k)
+
+    def near(shape):
+        ulps = torch.randint(-3, 4, shape, generator=g).float()
+        return 1.0 + 2.0 ** -8 - 2.0 ** -17 + ulps * 2.0 ** -23
+    a, b = near((m, k)), near((k, n))
+    scale = 8.0 / k
+    want = torch.softmax(torch.matmul(a.double(), b.double()) * scale, dim=-1)
+    got = matmul_softmax(a.cuda(), b.cuda(), logit_scale=scale).double().cpu()
+    err = float((got - want).norm() / want.norm())
+    assert err <= 2 * 8.0 * 2.0 ** -24 * (1 + 0.29 * math.sqrt(6 * k / 16 / 3)) + 5e-7, err

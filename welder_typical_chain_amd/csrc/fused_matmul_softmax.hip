@@ -164,15 +164,18 @@ __device__ inline uint32_t bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
 // f32 inputs on the bf16 matrix cores.  A f32 value x is the exact sum of
 // three bf16 values: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1 (8, 8
 // and the last 8 of its 24 significant bits; both differences are exact in
-// f32).  Of the nine partial products of a . b the six of order 2^-18 and
-// above are summed, in f32:
+// f32).  Of the nine partial products of a . b six are summed, in f32:
 //   a0 b0 + a0 b1 + a1 b0 + a1 b1 + a0 b2 + a2 b0;
-// what is left out is below 2^-26 |a b|, a quarter of the rounding of one f32
-// product.  Six bf16 MFMAs cost 6/16 of the f32 MFMAs of the same k, and
-// round the accumulator less often (6 times per 16 k, not 8), so the sums are
-// no further from the 64-bit ones than f32 MFMAs leave them (relative 2-norm
-// error of the outputs, N(0, 1) logits, 1024 x 1024 x 1024: 5.5e-7, with f32
-// MFMAs 1.1e-6).
+// left out are a1 b2 + a2 b1 + a2 b2: with |x1| <= 2^-8 and |x2| <= 2^-17 of an x
+// in [1, 2), up to 2^-24 |a b|, as much as one f32 product's rounding (reached near
+// a = b = 1.0039); over random mantissas 2^-27.5 in the mean square, of either sign.
+// Six bf16 MFMAs cost 6/16 of the f32 MFMAs of the same k, and round the
+// accumulator less often (6 times per 16 k, not 8).  Relative 2-norm error of the
+// outputs against 64 bits, K = 1024, here and with f32 MFMAs: N(0, 1) logits 5.2e-7,
+// 1.1e-6; operands U(0, 1), logits 8, 1.4e-6, 3.5e-6.  Operands that all lie within
+// some units of the worst mantissa, logits 8, 1.1e-6, 3.6e-7: there the two products
+// a1 b2 and a2 b1 would give 3.0e-7, for 5 (64 x 64 tiles) to 18 % (128 x 128) more
+// time in every call.
 //
 // Values that do not split: infinities, NaN and values that round to an infinite
 // x0 (x - x0 is then NaN or infinite, and so is an accumulator at the end), and
