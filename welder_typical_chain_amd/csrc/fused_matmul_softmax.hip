@@ -188,21 +188,19 @@ __device__ inline uint32_t bload4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
 // -------------------------------------------------------------------------
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
-// The least nonzero magnitude seen, as 2 * bits - 1, which puts zero last, and
-// the largest.
-struct Range {
+// The least nonzero magnitude seen: as 2 * bits - 1, which puts zero last.
+struct Tiny {
   uint32_t least = 0xFFFFFFFFu;
-  float most = 0.0f;
-  __device__ inline void see(uint32_t x, uint32_t y) {
-    least = min(least, min((x << 1) - 1u, (y << 1) - 1u));
-    most = fmaxf(fmaxf(most, fabsf(__builtin_bit_cast(float, x))), fabsf(__builtin_bit_cast(float, y)));
-  }
-  __device__ inline bool tiny() const { return least < (27u << 24) - 1u; }  // 2^-100
+  __device__ inline void see(uint32_t x, uint32_t y) { least = min(least, min((x << 1) - 1u, (y << 1) - 1u)); }
+  __device__ inline bool any() const { return least < (27u << 24) - 1u; }  // 2^-100
 };
 // K products, in each of which both values may have lost 2^-125 beside one of
-// magnitude `most`, move a logit (log2 units: c2 times the sum) by at most
+// the tile's largest magnitude, `most`, move a logit (log2 units: c2 times the sum) by at most
 // |c2| K 2^-124 most: 2^-36, a 4096th of an output's f32 rounding, while most is
 // below this over |c2| K.  Probabilities (2^-100 and less beside 1) stay below it.
+// `most` is looked for only in tiles with a tiny value, in a second pass over
+// the operands (1024 x 1024 x 1024 25 -> 28 us); kept beside `least` in the main
+// loop it took 2 % of every call.
 constexpr float kTinyMatters = 0x1p88f;
 
 // The three parts of the pair (x, y), each two packed bf16.
@@ -273,20 +271,32 @@ template <int TM, int NT> struct F32Regs {
 #pragma unroll
     for (int i = 0; i < V; ++i) b[i] = bload16(w.rb, off + (ok ? 16u * i : 0u));
   }
-  // Splits the values and writes their parts to the planes of a stage.
-  __device__ inline void store(uint8_t* stage, int t, Range& seen) const {
-    const int row = t / TPA, ak = (t % TPA) * E, bk = t / TPB, bn = (t % TPB) * E;
-    put(a, stage + a64_lds_offset(row, ak >> 3) + (ak & 7) * 2, Cfg<DT_F32, TM>::kAPlane, seen);
-    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_offset<TM>(bk, bn), Cfg<DT_F32, TM>::kBPlane, seen);
+  __device__ inline float largest() const {
+    float most = 0.0f;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u32x4 x = a[i], y = b[i];
+        const uint32_t xe = x[e], ye = y[e];
+        most = fmaxf(fmaxf(most, fabsf(__builtin_bit_cast(float, xe))), fabsf(__builtin_bit_cast(float, ye)));
+      }
+    return most;
   }
-  static __device__ inline void put(const u32x4 (&v)[V], uint8_t* dst, int plane, Range& seen) {
+  // Splits the values and writes their parts to the planes of a stage.
+  __device__ inline void store(uint8_t* stage, int t, Tiny& tiny) const {
+    const int row = t / TPA, ak = (t % TPA) * E, bk = t / TPB, bn = (t % TPB) * E;
+    put(a, stage + a64_lds_offset(row, ak >> 3) + (ak & 7) * 2, Cfg<DT_F32, TM>::kAPlane, tiny);
+    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_offset<TM>(bk, bn), Cfg<DT_F32, TM>::kBPlane, tiny);
+  }
+  static __device__ inline void put(const u32x4 (&v)[V], uint8_t* dst, int plane, Tiny& tiny) {
     u32x3 w[2 * V];
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       const u32x4 x = v[i];
-      seen.see(x[0], x[1]);
+      tiny.see(x[0], x[1]);
       w[2 * i] = split_pair(x[0], x[1]);
-      seen.see(x[2], x[3]);
+      tiny.see(x[2], x[3]);
       w[2 * i + 1] = split_pair(x[2], x[3]);
     }
 #pragma unroll
@@ -845,15 +855,12 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
     // some value of the tile: is tiny; is large enough for a tiny one to matter
     uint32_t* redo = reinterpret_cast<uint32_t*>(smem + L::RED_OFF);
     if (t < 2) redo[t] = 0u;
-    Range seen;
+    Tiny tiny;
     Regs R[PF];
 #pragma unroll
     for (int q = 0; q < PF; ++q) R[q].load(w, q);
-    // read here, under the first loads: the parameter block comes from memory
-    float reach = fabsf(p.c2) * (float)K32;
-    asm volatile("" : "+v"(reach));
     auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    R[0].store(smem, t, seen);
+    R[0].store(smem, t, tiny);
     R[0].load(w, PF);
     meet();
     auto iteration = [&](auto q_c, int kt) {
@@ -861,7 +868,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
       Frags F;
       F.read(smem + (kt & 1) * STAGE, lane, wm, nw, kg);
       F.products(acc);
-      R[(Q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE, t, seen);
+      R[(Q + 1) % PF].store(smem + ((kt + 1) & 1) * STAGE, t, tiny);
       R[(Q + 1) % PF].load(w, kt + 1 + PF);
       // The scheduler's order: the fragment reads, then the splitting spread
       // over the MFMAs.  In source order a wave would first issue its MFMAs,
@@ -888,8 +895,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         if (++kt == nk) break;
       }
     }
-    if (seen.tiny()) redo[0] = 1u;
-    if (seen.most * reach > kTinyMatters) redo[1] = 1u;
+    if (tiny.any()) redo[0] = 1u;
     uint32_t blocks = 0;  // the wave's blocks to recompute, bit mt * NTN + j
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -901,7 +907,18 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         blocks |= __all(fine) ? 0u : 1u << (mt * NTN + j);
       }
     meet();
-    if (redo[0] & redo[1]) blocks = (1u << (MT * NTN)) - 1u;
+    if (__builtin_expect(redo[0] != 0u, 0)) {
+      float most = 0.0f;
+      for (int kt = 0; kt < nk; kt += PF) {
+#pragma unroll
+        for (int q = 0; q < PF; ++q) R[q].load(w, kt + q);
+#pragma unroll
+        for (int q = 0; q < PF; ++q) most = fmaxf(most, R[q].largest());
+      }
+      if (most * fabsf(p.c2) * (float)K32 > kTinyMatters) redo[1] = 1u;
+      meet();
+      if (redo[1]) blocks = (1u << (MT * NTN)) - 1u;
+    }
     blocks = __builtin_amdgcn_readfirstlane(blocks);
     if (__builtin_expect(blocks != 0u, 0)) {
 #pragma unroll 1
