@@ -144,7 +144,7 @@ MEASURED_BEST = [
     ((1, 2048, 8192, 512, F16, F16), W256[F16], _lib.PATH_SPLIT),      # 40.1 vs 47.6
     ((8, 2048, 2048, 128, F16, F16), ROWS, _lib.PATH_ROWS),            # 50.3 vs split 54.3
     ((16, 512, 512, 64, F16, F16), T128[F16], _lib.PATH_EXCHANGE),     # 7.5 vs 8.0
-    ((1, 4096, 2048, 128, F16, F16), T256[F16], _lib.PATH_SPLIT),      # 22.2 vs 24.4
+    ((1, 4096, 2048, 128, F16, F16), LDR[F16], _lib.PATH_EXCHANGE),    # 14.1 vs split 22.3
     ((64, 2048, 2048, 128, F16, F16), ROWS, _lib.PATH_ROWS),           # C3: 250 vs 454
     ((1, 1024, 32768, 4096, BF16, BF16), W256[BF16], _lib.PATH_SPLIT),  # C4: 257 vs 293
     ((1, 8192, 8192, 4096, FP8, F16), W256[FP8], _lib.PATH_SPLIT),     # C5: 258 vs 347

@@ -21,14 +21,15 @@ def _plan(batch, m, n, k=256):
 
 
 def test_rule(native_lib):
-    """128-row tiles while they fit on 256 CUs, then 256-row tiles on at most
-    255 of them, for rows of at most 32 column tiles."""
+    """128-row tiles while they fit on 256 CUs, then 256-row tiles while those do,
+    for rows of at most 32 column tiles."""
     assert _plan(1, 2048, 2048)["grid"] == 256
     pl = _plan(1, 2049, 2048)
     assert pl["grid"] == 9 * 16 and pl["tiles"] == TILES
     assert _plan(1, 3840, 2048)["grid"] == 15 * 16
+    assert _plan(1, 4096, 2048)["grid"] == _plan(1, 2048, 4096)["grid"] == _plan(8, 1024, 1024)["grid"] == 256
     assert _plan(1, 1500, 4096)["grid"] == 6 * 32
-    for m, n in ((3841, 2048), (1500, 4104)):
+    for m, n in ((4097, 2048), (1500, 4104)):
         with pytest.raises(_lib.WtcError):
             _plan(1, m, n)
     # a slot per 128 rows: the entries fit what the workspace holds for them
@@ -39,6 +40,8 @@ def test_rule(native_lib):
 SHAPES = [
     # the last row block: 220 rows, 1 row, a full one; two row blocks per batch of 2 rows and 257
     (1, 1500, 3000, 1000), (1, 2049, 2048, 64), (1, 3840, 2048, 136), (15, 130, 2048, 256), (5, 257, 3080, 72),
+    # every CU: 256 tiles (with f32 outputs every slot there is)
+    (1, 4096, 2048, 72), (8, 1000, 1024, 128),
     # 32 column tiles, the last of 8 columns; no K at all
     (1, 1500, 3976, 320), (1, 2304, 2048, 0),
 ]
@@ -76,7 +79,7 @@ def test_tall_exchange(native_lib, batch, m, n, k, in_dtype, out_dtype):
 
 def test_slots_of_f32_outputs(native_lib):
     """Two entries a row (max and sum): four slots per tile, in the workspace and within the slots' limit."""
-    for m in (2049, 3840):
+    for m in (2049, 3840, 4096):
         pl = _lib.plan(1, m, 2048, 256, _lib.DTYPE_F16, _lib.DTYPE_F32, _lib.PATH_EXCHANGE)
         assert pl["grid"] == -(-m // 256) * 16 and 4 * pl["grid"] <= 1024
         assert pl["workspace_bytes"] >= 256 + 4096 + 4 * pl["grid"] * 1024

@@ -35,7 +35,7 @@ constexpr unsigned kSplitPaths = bit(WTC_PATH_SPLIT) | bit(WTC_PATH_UNFUSED);
 // The constants were fitted (least squares on the log of the time) to
 // back-to-back timings of every variant on every path over the 60 shapes
 // of calibrate.py on MI355X.  Fitted on three of its four shape sets and
-// scored on the fourth, in turn, the fused ranking lost 0.83 % on average
+// scored on the fourth, in turn, the fused ranking lost 0.78 % on average
 // against the measured fastest choice (the hand-written rules it replaces:
 // 5.3 %).
 struct TileCal {
@@ -45,10 +45,10 @@ struct TileCal {
 // [tile variant][0: 16-bit, 1: fp8, 2: f32, 3: f32 64 x 64]; fixed parts shared
 // across 16-bit and fp8 inputs.  Rows: kVarTile128, kVarTile128Loaders, kVarTile256, kVarTile256x256.
 const TileCal kTileCal[4][4] = {
-    /* kVarTile128 */ {{625.51, {2913.5, 4610.4, 0}}, {627.53, {2913.5, 4610.4, 0}}, {2187.18, {4978.1, 4978.1, 0}}, {593.59, {4509.2, 0, 0}}},
-    /* kVarTile128Loaders */ {{556.60, {3280.5, 5103.1, 254}}, {545.51, {3280.5, 5103.1, 254}}, {0, {0, 0, 0}}},
-    /* kVarTile256 */ {{1159.61, {0, 9359.9, 0}}, {1301.15, {0, 9359.9, 0}}, {0, {0, 0, 0}}},
-    /* kVarTile256x256 */ {{2020.66, {0, 17970.4, 6164}}, {1698.44, {0, 17970.4, 6164}}, {0, {0, 0, 0}}},
+    /* kVarTile128 */ {{632.66, {3188.1, 4614.2, 0}}, {635.88, {3188.1, 4614.2, 0}}, {2190.53, {5134.5, 5134.5, 0}}, {595.42, {4799.6, 0, 0}}},
+    /* kVarTile128Loaders */ {{563.64, {3558.8, 5107.3, 254}}, {553.73, {3558.8, 5107.3, 254}}, {0, {0, 0, 0}}},
+    /* kVarTile256 */ {{1161.14, {0, 9481.9, 0}}, {1280.80, {0, 9481.9, 0}}, {0, {0, 0, 0}}},
+    /* kVarTile256x256 */ {{2036.50, {0, 18296.2, 6164}}, {1693.92, {0, 18296.2, 6164}}, {0, {0, 0, 0}}},
 };
 int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // Rows kernel, cycles per row block: a fixed part, and one per 128-column tile
@@ -56,7 +56,7 @@ int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // 128 rows of f32 outputs add (14 shapes of 12 to 84 row blocks took 15 to 50 % more
 // than modelled without it: 37 x 152 x 1952 x 128 f16 58.6 us, 43.8 with 256-row
 // tiles; 296 x 4 x 5192 x 96, 4 rows stored, does not: 166, split 236).
-constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4516.7, kRowsTile4Cyc = 3212.1, kRowsTileF32Cyc = 1700.0;
+constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4517.5, kRowsTile4Cyc = 3214.1, kRowsTileF32Cyc = 1700.0;
 // Few-row kernel: a workgroup's first loads and its softmax (us), one 16 KiB unit
 // of B (us), and the rate at which all workgroups together read B (GB/s): read
 // off 36 timings of 4 to 512 batches x 1 to 16 rows x 256 to 7936 columns (not
@@ -71,8 +71,8 @@ constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFe
 // last tile of a row block: fixed (us) and per column tile (us); the HBM
 // rate of the fused paths' streaming passes and the chip-wide rate that
 // prices k-tile bytes (GB/s).
-constexpr double kLaunchUs = 3.9636, kExchangeUs = 0.3687, kExchangePerTileUs = 0.11020;
-constexpr double kHbmGBs = 6615.1, kFeedGBs = 115179.1;
+constexpr double kLaunchUs = 3.9550, kExchangeUs = 0.2502, kExchangePerTileUs = 0.10301;
+constexpr double kHbmGBs = 6623.8, kFeedGBs = 122654.6;
 // A 256 x 256 tile of f32 outputs takes this much longer (its second staging round
 // and stores; fp8 4 x 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles).  With
 // eight k-tiles or more it is left out: the 128-column tiles then lose as much,
@@ -154,7 +154,7 @@ bool variant_by_id(int in_dt, int id, VariantDesc* out) {
 static bool tall_exchange(const VariantDesc& v, const Problem& p) {
   if (v.id != kVarTile128Loaders) return false;
   const int64_t nT = cdiv(p.n, 128), tiles = p.batch * cdiv(p.m, 256) * nT;
-  return p.batch * cdiv(p.m, 128) * nT > (int64_t)p.cu_count * std::max(1, p.xch_per_cu) && tiles < p.cu_count &&
+  return p.batch * cdiv(p.m, 128) * nT > (int64_t)p.cu_count * std::max(1, p.xch_per_cu) && tiles <= p.cu_count &&
          nT <= kTallMaxColTiles && tall_slots(p.out_dt) * tiles <= kExchangeMaxTiles;
 }
 

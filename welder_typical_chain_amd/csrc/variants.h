@@ -81,13 +81,14 @@ constexpr int kF32SmallTilesPerCu = 2;
 constexpr int64_t kF32OneGroupK = 192;
 // And 16-bit or fp8 inputs on the exchange path when 128-row tiles outnumber the
 // CUs and 256-row tiles (the loader-wave variant's request, run without loader
-// waves) do not.  They leave CUs idle, as they do on the split path, but need no
-// second pass over the output (us, split and exchange: 1500 x 3000 x 1000 bf16
+// waves) do not.  They may leave CUs idle, as they do on the split path, but need
+// no second pass over the output (us, split and exchange: 1500 x 3000 x 1000 bf16
 // 27.7, 24.5; 3328 x 2048 x 512 f16 25.2, 17.4; 15 x 130 x 2048 x 256 bf16 -> f32
-// 23.9, 15.2; 2304 x 2048 x 1024 fp8 23.9, 18.5).  Rows of more than 32 column
-// tiles stay on the split path: a thread would poll a second group of entries
-// (1000 x 4104 x 2064 fp8, 33 tiles: split 31.3, exchange 34.0); and so does a
-// grid that takes every CU, whose plan is pinned (4096 x 2048 x 128, split).
+// 24.1, 16.1; 2304 x 2048 x 1024 fp8 23.9, 18.5; a tile on every CU: 4096 x 2048 x
+// 128 f16 22.3, 14.2, x 1024 32.0, 28.6, 8 x 1024 x 1024 x 512 31.5, 18.8, 4096 x
+// 2048 x 4096 fp8 46.9, 43.8; of 30 such calls timed none was slower).  Rows of
+// more than 32 column tiles stay on the split path: a thread would poll a second
+// group of entries (1000 x 4104 x 2064 fp8, 33 tiles: split 31.3, exchange 34.0).
 constexpr int64_t kTallMaxColTiles = 32;
 // Exchange slots such a tile takes: one per 128 rows and, with f32 outputs, two
 // (the row's max and its sum).
