@@ -86,3 +86,27 @@ def test_ranking_generalises_to_held_out_sets(records):
         losses += list(calibrate.ranking_losses(x, [r for r in records if r["set"] == held]).values())
     assert sum(losses) / len(losses) < 0.02
     assert max(losses) < 0.2
+
+
+# Calls that lost 10 to 25 % to the former choice while B rows off the cache
+# lines, f32 outputs and f32 inputs on the split path were not priced: (batch, m, n,
+# k, in, out), the measured fastest choice, its us and the other choice's.
+LOADERS, W64X32, ROWS128 = [128, 128, 64, 2, 32], [128, 128, 64, 2, 16], [128, 128, 128, 2, 16]
+TALL, F32_TILES = [256, 128, 64, 2, 32], [128, 128, 32, 2, 32]
+PRICED = [
+    ((1, 943, 17592, 1984, "f16", "f32"), LOADERS, "split"),       # 128, 160 (276 tiles of 256 x 256)
+    ((1, 1303, 4616, 1536, "bf16", "bf16"), TALL, "split"),        # 37.5, 44.5
+    ((24, 458, 264, 64, "bf16", "f32"), ROWS128, "rows"),          # 10.7, 13.3
+    ((12, 1754, 248, 128, "bf16", "f32"), ROWS128, "rows"),        # 12.1, 14.8
+    ((25, 287, 984, 80, "f16", "f32"), ROWS128, "rows"),           # 25.8, 33.1
+    ((6, 1919, 264, 128, "bf16", "bf16"), ROWS128, "rows"),        # 11.5, 12.8
+    ((2, 117, 7576, 272, "bf16", "f32"), W64X32, "exchange"),      # 12.3, 14.3
+    ((1, 602, 2296, 64, "f32", "f32"), F32_TILES, "exchange"),     # 11.7, 16.7
+]
+
+
+@pytest.mark.parametrize("shape,tiles,path", PRICED)
+def test_unaligned_rows_and_f32_outputs_are_priced(native_lib, shape, tiles, path):
+    batch, m, n, k, in_dt, out_dt = shape
+    pl = _lib.plan(batch, m, n, k, CODES[in_dt], CODES[out_dt], _lib.PATH_AUTO, None, 256, 1)
+    assert (pl["tiles"], pl["path"]) == (tiles, PATHS[path])

@@ -198,15 +198,19 @@ _SCALARS = ["launch_us", "exchange_us", "exchange_per_tile_us", "hbm_gbs", "feed
             "rows_block_cyc", "rows_tile_cyc", "rows_tile4_cyc"]
 
 
-# 128-column tiles of more than two waves: what they re-read of A and B
+# Parts that are not fitted to the table (csrc/variants.cpp says what they are
+# read off).  128-column tiles of more than two waves: what they re-read of A and B
 MANY_WAVES = 1.1
-# a 256 x 256 tile of f32 outputs: its second staging round and store, with
-# fewer than eight k-tiles
-WIDE_F32_CYC = 17000.0
+# lines fetched beyond its own for a k-row of B that does not start on a cache line
+UNALIGNED_LINES = 2.5
+# a 256 x 256 tile of f32 outputs: its second staging round and stores
+WIDE_F32_CYC = 7000.0
 # a row block's column tile of f32 outputs, all 128 rows stored
-ROWS_TILE_F32_CYC = 1700.0
-# a 256 x 128 tile's fixed part on the exchange path
-TALL_FIXED_CYC = 11000.0
+ROWS_TILE_F32_CYC = 1500.0
+# a 256 x 128 tile's fixed part on the exchange path, and what f32 outputs add
+TALL_FIXED_CYC, TALL_F32_CYC = 11500.0, 2300.0
+# f32 inputs: two 64 x 64 tiles at once on a CU, the split path's tile pass
+F32_PAIR_SHARE, F32_SPLIT_US = 0.75, 2.6
 
 
 def _clock_ghz(busy):
@@ -254,20 +258,24 @@ def model_us(x, r, cu=256):
             # more, and with 256 x 256 tiles, at the mean one
             own = tiles <= 2 * cu and v != 4
             f = _clock_ghz(active / cu if own else tiles / (math.ceil(tiles / cu) * cu))
-            per_kt = kt[(2 if tall else v, cls)] + (rows + cols) * 128 * active * f / c["feed_gbs"]
+            lines = UNALIGNED_LINES * 128 / isz if n * isz % 128 else 0.0
+            per_kt = kt[(2 if tall else v, cls)] + (rows + cols + lines) * 128 * active * f / c["feed_gbs"]
             fixed = fx[(v, 1, 2) if cls == 2 else (v, epi, 3 if cls == 3 else 0)]
             if tall:
-                fixed = TALL_FIXED_CYC
-            if v == 4 and r["out"] == "f32" and nk < 8:
+                fixed = TALL_FIXED_CYC + (TALL_F32_CYC if osz == 4 else 0.0)
+            if v == 4 and osz == 4:
                 fixed += WIDE_F32_CYC
             t_tiles += count * (fixed + nk * per_kt) / (f * 1e3)
     if tiles > 2 * cu and v != 4:
         t_tiles *= MANY_WAVES
+    if cls == 3 and tiles > cu:
+        t_tiles *= F32_PAIR_SHARE
     if r["path"] == "exchange":
         t_xch = c["exchange_us"] + c["exchange_per_tile_us"] * n_t if n > cols else 0.0
         return c["launch_us"] + max(t_tiles, (ab + elems * osz) * us_per_byte) + t_xch
     stats = b * m * n_t * 8
-    return (2 * c["launch_us"] + max(t_tiles, (ab + elems * osz + stats) * us_per_byte)
+    f32_us = F32_SPLIT_US if r["in"] == "f32" else 0.0
+    return (f32_us + 2 * c["launch_us"] + max(t_tiles, (ab + elems * osz + stats) * us_per_byte)
             + (2 * elems * osz + stats) * us_per_byte)
 
 

@@ -45,10 +45,10 @@ struct TileCal {
 // [tile variant][0: 16-bit, 1: fp8, 2: f32, 3: f32 64 x 64]; fixed parts shared
 // across 16-bit and fp8 inputs.  Rows: kVarTile128, kVarTile128Loaders, kVarTile256, kVarTile256x256.
 const TileCal kTileCal[4][4] = {
-    /* kVarTile128 */ {{632.66, {3188.1, 4614.2, 0}}, {635.88, {3188.1, 4614.2, 0}}, {2190.53, {5134.5, 5134.5, 0}}, {595.42, {4799.6, 0, 0}}},
-    /* kVarTile128Loaders */ {{563.64, {3558.8, 5107.3, 254}}, {553.73, {3558.8, 5107.3, 254}}, {0, {0, 0, 0}}},
-    /* kVarTile256 */ {{1161.14, {0, 9481.9, 0}}, {1280.80, {0, 9481.9, 0}}, {0, {0, 0, 0}}},
-    /* kVarTile256x256 */ {{2036.50, {0, 18296.2, 6164}}, {1693.92, {0, 18296.2, 6164}}, {0, {0, 0, 0}}},
+    /* kVarTile128 */ {{629.84, {3269.7, 4715.4, 0}}, {632.56, {3269.7, 4715.4, 0}}, {2169.61, {2450.2, 2450.2, 0}}, {755.79, {4185.3, 0, 0}}},
+    /* kVarTile128Loaders */ {{560.75, {3641.3, 5208.9, 254}}, {550.35, {3641.3, 5208.9, 254}}, {0, {0, 0, 0}}},
+    /* kVarTile256 */ {{1153.19, {0, 9714.1, 0}}, {1272.56, {0, 9714.1, 0}}, {0, {0, 0, 0}}},
+    /* kVarTile256x256 */ {{2026.70, {0, 18521.3, 6164}}, {1694.63, {0, 18521.3, 6164}}, {0, {0, 0, 0}}},
 };
 int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // Rows kernel, cycles per row block: a fixed part, and one per 128-column tile
@@ -56,7 +56,7 @@ int cal_row(int id) { return id == kVarTile256x256 ? 3 : id; }
 // 128 rows of f32 outputs add (14 shapes of 12 to 84 row blocks took 15 to 50 % more
 // than modelled without it: 37 x 152 x 1952 x 128 f16 58.6 us, 43.8 with 256-row
 // tiles; 296 x 4 x 5192 x 96, 4 rows stored, does not: 166, split 236).
-constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4517.5, kRowsTile4Cyc = 3214.1, kRowsTileF32Cyc = 1700.0;
+constexpr double kRowsBlockCyc = 2100.0, kRowsTileCyc = 4520.9, kRowsTile4Cyc = 3223.4, kRowsTileF32Cyc = 1500.0;
 // Few-row kernel: a workgroup's first loads and its softmax (us), one 16 KiB unit
 // of B (us), and the rate at which all workgroups together read B (GB/s): read
 // off 36 timings of 4 to 512 batches x 1 to 16 rows x 256 to 7936 columns (not
@@ -71,18 +71,31 @@ constexpr double kFewFixedUs = 1.5, kFewUnitUs = 0.245, kFewHbmGBs = 6000.0, kFe
 // last tile of a row block: fixed (us) and per column tile (us); the HBM
 // rate of the fused paths' streaming passes and the chip-wide rate that
 // prices k-tile bytes (GB/s).
-constexpr double kLaunchUs = 3.9550, kExchangeUs = 0.2502, kExchangePerTileUs = 0.10301;
-constexpr double kHbmGBs = 6623.8, kFeedGBs = 122654.6;
-// A 256 x 256 tile of f32 outputs takes this much longer (its second staging round
-// and stores; fp8 4 x 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles).  With
-// eight k-tiles or more it is left out: the 128-column tiles then lose as much,
-// unmodelled, to B rows that do not start on a cache line (fp8 524 x 51576 x 6816:
-// 256 x 256 tiles 337 us, 128 x 128 547; f16 638 x 40776 x 2368 189, 274).
-constexpr double kManyWaves = 1.1, kWideF32Cyc = 17000.0, kWideF32KTiles = 8.0;
+constexpr double kLaunchUs = 3.9154, kExchangeUs = 0.2854, kExchangePerTileUs = 0.09870;
+constexpr double kHbmGBs = 6776.6, kFeedGBs = 117314.0;
+// The parts below are not in the fit (the table has few f32 outputs and few B
+// rows that do not start on a cache line): read off the timings of 6000 drawn
+// calls, every choice of each (16-bit and fp8 general products, attention, logits),
+// so that few calls lose to the choice before the fit (16 by more than 3 %, 3 by
+// more than 10 %; without them 29 and 14) and the picks lose 1.6 % on average
+// against the fastest (2.0).
+// k-rows of B that do not start on a cache line: lines fetched beyond the row's
+// own (bf16 1303 x 4616 x 1536, 407 tiles of 128 x 128: 44.5 us, priced 36.0 without
+// this, 37.7 with; 222 of 256 x 128 37.5, priced 37.1.  Tiles of 256 columns pay half as much per column).
+constexpr double kUnalignedLines = 2.5;
+// A 256 x 256 tile of f32 outputs: its second staging round and stores (fp8 4 x
+// 1015 x 4488 x 400: 79.7 us, 60.1 with 128 x 128 tiles; f16 943 x 17592 x 1984,
+// 276 tiles: 160, 128 with 128 x 128).
+constexpr double kManyWaves = 1.1, kWideF32Cyc = 7000.0;
 // A 256 x 128 tile's fixed part on the exchange path (its k-tiles cost what the split
-// path's do): read off three timings (modelled and measured us: 1536 x 4096 x 1024
-// bf16 25.6, 24.8; 2560 x 2560 x 1024 f16 24.7, 23.9; 2 x 1536 x 1536 x 512 16.2, 16.5).
-constexpr double kTallFixedCyc = 11000.0;
+// path's do), and what f32 outputs add (twice the entries and stores): modelled and
+// measured us: 1536 x 4096 x 1024 bf16 25.3, 24.8; 4096 x 2048 x 512 f16 20.5, 19.8,
+// to f32 22.0, 23.7; 12 x 1754 x 248 x 128 bf16 to f32 13.0, 14.8 (rows kernel 12.1).
+constexpr double kTallFixedCyc = 11500.0, kTallF32Cyc = 2300.0;
+// f32 inputs: two 64 x 64 tiles on a CU at once take this part of one after the
+// other; the split path's tile pass takes this much longer (us) than the exchange
+// path's on the same tiles (602 x 2296 x 64: 11.7 us, split 16.7).
+constexpr double kF32PairShare = 0.75, kF32SplitUs = 2.6;
 // Unfused row passes (one 256-thread workgroup per row, eight per CU): HBM
 // rate, and the rate one workgroup streams its row at (GB/s).
 constexpr double kRowPassHbmGBs = 5293.0, kRowPassWgGBs = 5.573;
@@ -266,7 +279,9 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
   const int epi = path == WTC_PATH_EXCHANGE ? 0 : (path == WTC_PATH_SPLIT ? 1 : 2);
   const double tiles = (double)variant_grid(v, path, p);
   const double nk = (double)cdiv(p.k * in_bytes(p.in_dt), 128);
-  const double kt_bytes = (double)(ts.rows + ts.cols) * 128.0;  // A and B per 128 bytes of K
+  // A and B per 128 bytes of K
+  const bool unaligned = p.n * in_bytes(p.in_dt) % 128 != 0;
+  const double kt_bytes = (ts.rows + ts.cols + (unaligned ? kUnalignedLines * 128.0 / isz : 0.0)) * 128.0;
   auto wave_us = [&](double active) {
     // One full wave and a part of another: each at its own clock (fp8 1000 x 4104
     // x 2064, 264 tiles of 128 x 128: 35.2 us, where the mean clock gave 26 and
@@ -275,9 +290,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     const bool own = tiles <= 2 * cu && v.id != kVarTile256x256;
     const double f = clock_ghz(own ? active / cu : tiles / (std::ceil(tiles / cu) * cu));
     const double kt = cal.kt_cyc + kt_bytes * active * f / kFeedGBs;
-    const bool wide = v.id == kVarTile256x256 && epi == 1 && osz == 4 && nk < kWideF32KTiles;
-    const double wide_f32 = wide ? kWideF32Cyc : 0.0;
-    const double fixed = tall ? kTallFixedCyc : cal.fixed_cyc[epi];
+    const double wide_f32 = v.id == kVarTile256x256 && epi == 1 && osz == 4 ? kWideF32Cyc : 0.0;
+    const double fixed = tall ? kTallFixedCyc + (osz == 4 ? kTallF32Cyc : 0.0) : cal.fixed_cyc[epi];
     return (fixed + wide_f32 + nk * kt) / (f * 1e3);
   };
   const double full = std::floor(tiles / cu), rem = tiles - full * cu;
@@ -285,7 +299,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
   // above say: without this part a row of 145 of them was put before 73 tiles of
   // 256 x 256 (bf16 607 x 18520 x 2240: 101 us, 70 with the latter).
   const double many = tiles > 2 * cu && v.id != kVarTile256x256 ? kManyWaves : 1.0;
-  const double t_tiles = many * (full * wave_us(cu) + (rem > 0 ? wave_us(rem) : 0.0));
+  const double pair = ts.rows == 64 && tiles > cu ? kF32PairShare : 1.0;
+  const double t_tiles = many * pair * (full * wave_us(cu) + (rem > 0 ? wave_us(rem) : 0.0));
   if (path == WTC_PATH_EXCHANGE) {
     const double t_hbm = (ab_bytes + elems * osz) * us_per_byte;
     const double t_xch = p.n > ts.cols ? kExchangeUs + kExchangePerTileUs * nT : 0.0;
@@ -297,7 +312,8 @@ double estimate_us(const VariantDesc& v, int path, const Problem& p) {
     const double stats = (double)p.batch * (double)p.m * nT * 8.0;
     const double t_hbm = (ab_bytes + elems * osz + stats) * us_per_byte;
     const double t_rescale = (2.0 * elems * osz + stats) * us_per_byte;
-    return 2 * kLaunchUs + std::max(t_tiles, t_hbm) + t_rescale;
+    const double f32 = p.in_dt == WTC_DTYPE_F32 ? kF32SplitUs : 0.0;
+    return 2 * kLaunchUs + std::max(t_tiles, t_hbm) + t_rescale + f32;
   }
   // unfused: f32 logits, then max, exp, sum and divide passes over them,
   // each at the HBM rate or, with few rows, at the rate of its workgroups
