@@ -2,14 +2,11 @@
 // of one k-slab of chain_wide_kernel's 256x256 tile).
 //
 // Uses the kernel's own index maps (welder_typical_chain_amd/csrc/tile_layout.h)
-// to move one k-tile of A and B from "HBM" through the register transpose into
-// the LDS stage, read the MFMA fragments back, run a reference model of the
-// 32x32xK MFMA (lane l supplies row/column l%32 and k-group l/32; register v of
-// the result holds D[8*(v/4) + 4*(l/32) + v%4][l%32]), and map the
-// accumulators to output coordinates the way the epilogue does.  Values are
-// small integers so the products are exact; the result must equal the plain
-// integer matmul.  Also checks that every LDS byte of the stage is written
-// exactly once, that the XCD remap is a bijection, and counts LDS bank
+// to move one k-tile of A and B from "HBM" into the LDS stage and read the MFMA
+// fragments back: 16-bit and fp8 tiles (direct-to-LDS loads), the bf16 planes of
+// f32 tiles, the 256x256 tiles (with a reference model of the MFMA).  Also checks
+// that every LDS byte of the stage is written exactly once, that the XCD remap
+// is a bijection, and counts LDS bank
 // conflicts (64 banks x 4 bytes, 16 lanes per 128-bit access phase).  Also
 // replays the row-block kernel's pass-2 output hand-off through its LDS out
 // stage (run_rows_out).
@@ -48,145 +45,86 @@ struct Conflicts {
   }
 };
 
-static int64_t elem(const std::vector<uint8_t>& buf, size_t off, int sz) {
-  if (sz == 1) return buf[off];
-  if (sz == 2) { uint16_t x; std::memcpy(&x, buf.data() + off, 2); return x; }
-  uint32_t x; std::memcpy(&x, buf.data() + off, 4); return x;
-}
-
-static void run(int sz, const char* name) {
-  const int KE = kKTileBytes / sz;  // elements of K in one k-tile
-  const int EPC = kChunkBytes / sz;
-  // global tiles with small distinct-ish integer values
-  std::vector<uint8_t> A((size_t)BM * kKTileBytes), B((size_t)KE * BN * sz);
-  for (int m = 0; m < BM; ++m)
-    for (int k = 0; k < KE; ++k) {
-      uint32_t v = (uint32_t)((m * 7 + k * 3) % 13 + 1);
-      std::memcpy(A.data() + (size_t)m * kKTileBytes + k * sz, &v, sz);
-    }
-  for (int k = 0; k < KE; ++k)
-    for (int n = 0; n < BN; ++n) {
-      uint32_t v = (uint32_t)((k * 5 + n * 11) % 17 + 1);
-      std::memcpy(B.data() + ((size_t)k * BN + n) * sz, &v, sz);
-    }
-  const int A_STAGE = BM * kKTileBytes;
-  std::vector<uint8_t> lds((size_t)A_STAGE + BN * kKTileBytes, 0);
-  std::vector<int> cover(lds.size(), 0);
-  Conflicts cw_a, cw_b, cr_a, cr_b;
-
-  // ---- A: all 256 threads, 4 passes of one 16-byte chunk each
-  for (int j = 0; j < 4; ++j)
-    for (int wave = 0; wave < 4; ++wave)
-      for (int ph = 0; ph < 4; ++ph) {
-        std::vector<int> addrs;
-        for (int l = ph * 16; l < ph * 16 + 16; ++l) {
-          const int t = wave * 64 + l;
-          const int row = a_load_row(t, j), c = a_load_chunk(t);
-          const int off = a_lds_offset(row, c);
-          addrs.push_back(off);
-          std::memcpy(lds.data() + off, A.data() + (size_t)row * kKTileBytes + c * 16, 16);
-          for (int b = 0; b < 16; ++b) cover[off + b]++;
-        }
-        cw_a.phase(addrs, 16);
-      }
-  // ---- B: all 256 threads transpose an (EPC k) x 4 block into 4 chunks
-  for (int c = 0; c < 4; ++c)
-    for (int wave = 0; wave < 4; ++wave)
-      for (int ph = 0; ph < 4; ++ph) {
-        std::vector<int> addrs;
-        for (int l = ph * 16; l < ph * 16 + 16; ++l) {
-          const int t = wave * 64 + l;
-          const int g = b_load_colgroup(t), kc = b_load_chunkrow(t);
-          // the loader's k-rows as 16 row-major words, 4 columns per row
-          uint32_t words[16];
-          const int rows = EPC, row_bytes = 4 * sz;
-          for (int r = 0; r < rows; ++r)
-            std::memcpy(reinterpret_cast<uint8_t*>(words) + r * row_bytes,
-                        B.data() + ((size_t)(kc * EPC + r) * BN + 4 * g) * sz, row_bytes);
-          auto rw = [&](int i) { return words[i]; };
-          uint32_t unit[4];
-          for (int w = 0; w < 4; ++w) unit[w] = b_unit_word(rw, sz, c, w);
-          const int off = A_STAGE + b_lds_offset(kc, 4 * g + c, BN);
-          addrs.push_back(off);
-          std::memcpy(lds.data() + off, unit, 16);
-          for (int b = 0; b < 16; ++b) cover[off + b]++;
-        }
-        cw_b.phase(addrs, 16);
-      }
-  for (size_t i = 0; i < cover.size(); ++i)
-    CHECK(cover[i] == 1, "[%s] LDS byte %zu written %d times\n", name, i, cover[i]);
-
-  // ---- fragments + reference MFMA
-  std::vector<int64_t> acc(4 * 4 * 64 * 16, 0);  // [wave][mt*2+nt][lane][v]
-  auto ACC = [&](int wave, int mt, int nt, int l, int v) -> int64_t& {
-    return acc[(((size_t)wave * 4 + mt * 2 + nt) * 64 + l) * 16 + v];
-  };
-  const int steps = kChunksPerKTile / 2;  // chunk pairs per k-tile
-  for (int wave = 0; wave < 4; ++wave) {
-    const int wm = wave >> 1, wn = wave & 1;
-    for (int s = 0; s < steps; ++s) {
-      // operand bytes per lane: [lane][16]
-      std::vector<std::vector<uint8_t>> af(2, std::vector<uint8_t>(64 * 16)), bf(2, std::vector<uint8_t>(64 * 16));
-      for (int mt = 0; mt < 2; ++mt)
-        for (int ph = 0; ph < 4; ++ph) {
-          std::vector<int> addrs;
-          for (int l = ph * 16; l < ph * 16 + 16; ++l) {
-            const int off = a_lds_offset(wm * 64 + mt * 32 + frag_row(l), frag_chunk(l, s));
-            addrs.push_back(off);
-            std::memcpy(&af[mt][l * 16], lds.data() + off, 16);
-          }
-          cr_a.phase(addrs, 16);
-        }
-      for (int nt = 0; nt < 2; ++nt)
-        for (int ph = 0; ph < 4; ++ph) {
-          std::vector<int> addrs;
-          for (int l = ph * 16; l < ph * 16 + 16; ++l) {
-            const int off = A_STAGE + b_lds_offset(frag_chunk(l, s), wn * 64 + nt * 32 + frag_row(l), BN);
-            addrs.push_back(off);
-            std::memcpy(&bf[nt][l * 16], lds.data() + off, 16);
-          }
-          cr_b.phase(addrs, 16);
-        }
-      // D = X . Y with X = B^T fragment (rows i <- lane%32), Y = A^T fragment
-      for (int mt = 0; mt < 2; ++mt)
-        for (int nt = 0; nt < 2; ++nt) {
-          int64_t D[32][32] = {};
-          for (int i = 0; i < 32; ++i)
-            for (int j = 0; j < 32; ++j)
-              for (int g = 0; g < 2; ++g)
-                for (int e = 0; e < EPC; ++e)
-                  D[i][j] += elem(bf[nt], (size_t)(i + 32 * g) * 16 + e * sz, sz) *
-                             elem(af[mt], (size_t)(j + 32 * g) * 16 + e * sz, sz);
-          for (int l = 0; l < 64; ++l)
-            for (int v = 0; v < 16; ++v) ACC(wave, mt, nt, l, v) += D[acc_i(l, v)][acc_j(l)];
-        }
+// The bf16 planes of a f32 tile (tm x tm, threads nt): what each thread stores
+// (F32Regs) and each MFMA wave reads (F32Frags).  Every byte of a plane is
+// written once, and each lane's A and B operands are the same 8 consecutive k of
+// its row and its column.
+static void run_f32(int tm, int nt) {
+  const int e = tm * 32 / nt;
+  char name[32];
+  std::snprintf(name, sizeof name, "f32 %dx%d/%d", tm, tm, nt);
+  std::vector<uint16_t> A(tm * 32), B(32 * tm);
+  for (int i = 0; i < tm * 32; ++i) A[i] = (uint16_t)(i + 1), B[i] = (uint16_t)(i + 7);
+  std::vector<uint8_t> sa(tm * 64), sb(tm * 64);
+  std::vector<int> ca(sa.size(), 0), cb(sb.size(), 0);
+  Conflicts cw, cr_a, cr_b;
+  std::vector<int> wa, wb;
+  for (int t = 0; t < nt; ++t) {
+    const int oa = f32_a_store(t, e), ob = f32_b_store(t, e, tm);
+    CHECK(oa >= 0 && oa + 2 * e <= tm * 64 && ob >= 0 && ob + 2 * e <= tm * 64, "[%s] thread %d off the plane\n", name, t);
+    std::memcpy(&sa[oa], &A[f32_a_row(t, e) * 32 + f32_a_k(t, e)], 2 * e);
+    std::memcpy(&sb[ob], &B[f32_b_k(t, e, tm) * tm + f32_b_n(t, e, tm)], 2 * e);
+    for (int x = 0; x < 2 * e; ++x) ca[oa + x]++, cb[ob + x]++;
+    wa.push_back(oa);
+    wb.push_back(ob);
+    if ((int)wa.size() == 128 / e) {  // lanes that store 256 bytes
+      cw.phase(wa, 2 * e);
+      cw.phase(wb, 2 * e);
+      wa.clear();
+      wb.clear();
     }
   }
-  // ---- epilogue coordinates vs the plain matmul
-  std::vector<int> seen(BM * BN, 0);
-  for (int wave = 0; wave < 4; ++wave) {
-    const int wm = wave >> 1, wn = wave & 1;
-    for (int mt = 0; mt < 2; ++mt)
-      for (int nt = 0; nt < 2; ++nt)
+  for (size_t i = 0; i < ca.size(); ++i) CHECK(ca[i] == 1 && cb[i] == 1, "[%s] byte %zu of a plane\n", name, i);
+  const int half = tm / 2;  // 2 x 2 waves
+  for (int wave = 0; wave < 4; ++wave)
+    for (int s = 0; s < 2; ++s)
+      for (int sub = 0; sub < half; sub += 32) {
+        const int r0 = (wave >> 1) * half + sub, n0 = (wave & 1) * half + sub;
+        uint16_t aop[64][8], bop[64][8];
+        std::vector<int> addrs;
+        for (int l = 0; l < 64; ++l) {
+          const int off = a64_lds_offset(r0 + frag_row(l), frag64_chunk16(l, s));
+          std::memcpy(aop[l], &sa[off], 16);
+          addrs.push_back(off);
+          if ((l & 15) == 15) {
+            cr_a.phase(addrs, 16);
+            addrs.clear();
+          }
+        }
+        for (int h = 0; h < 2; ++h) {
+          uint16_t src[64][4];
+          for (int l = 0; l < 64; ++l) {
+            const int off = f32_b_offset(tm, btr_k(s, h, l), btr_n(n0, l));
+            std::memcpy(src[l], &sb[off], 8);
+            addrs.push_back(off);
+            if ((l & 31) == 31) {
+              cr_b.phase(addrs, 8);
+              addrs.clear();
+            }
+          }
+          for (int l = 0; l < 64; ++l)  // the transpose, as in run_dma16
+            for (int r = 0; r < 4; ++r) bop[l][4 * h + r] = src[16 * (l / 16) + 4 * r + (l % 16) / 4][(l % 16) % 4];
+        }
+        for (int l = 0; l < 64; ++l)
+          for (int x = 0; x < 8; ++x) {
+            const int k = 16 * s + 8 * (l >> 5) + x;
+            CHECK(aop[l][x] == A[(r0 + (l & 31)) * 32 + k], "[%s] A operand lane %d elem %d\n", name, l, x);
+            CHECK(bop[l][x] == B[k * tm + n0 + (l & 31)], "[%s] B operand lane %d elem %d\n", name, l, x);
+          }
+      }
+  // the accumulators' places in the tile: each once, four columns in a run
+  std::vector<int> seen(tm * tm, 0);
+  for (int wave = 0; wave < 4; ++wave)
+    for (int mt = 0; mt < half; mt += 32)
+      for (int n = 0; n < half; n += 32)
         for (int l = 0; l < 64; ++l)
           for (int v = 0; v < 16; ++v) {
-            const int m = wm * 64 + mt * 32 + acc_j(l);
-            const int n = wn * 64 + nt * 32 + acc_i(l, v);
-            seen[m * BN + n]++;
-            int64_t ref = 0;
-            for (int k = 0; k < KE; ++k)
-              ref += elem(A, (size_t)m * kKTileBytes + k * sz, sz) * elem(B, ((size_t)k * BN + n) * sz, sz);
-            CHECK(ACC(wave, mt, nt, l, v) == ref, "[%s] C[%d][%d] = %lld, want %lld\n", name, m, n,
-                  (long long)ACC(wave, mt, nt, l, v), (long long)ref);
-            if ((v & 3) != 0)
-              CHECK(acc_i(l, v) == acc_i(l, v & ~3) + (v & 3), "[%s] staging run not contiguous\n", name);
+            seen[((wave >> 1) * half + mt + acc_j(l)) * tm + (wave & 1) * half + n + acc_i(l, v)]++;
+            CHECK(acc_i(l, v) == acc_i(l, v & ~3) + (v & 3), "[%s] staging run not contiguous\n", name);
           }
-  }
-  for (int i = 0; i < BM * BN; ++i) CHECK(seen[i] == 1, "[%s] output %d covered %d times\n", name, i, seen[i]);
-  std::printf("[%s] lds bank-conflict ways: A write %d, B write %d, A read %d, B read %d\n", name,
-              cw_a.worst, cw_b.worst, cr_a.worst, cr_b.worst);
+  for (int i = 0; i < tm * tm; ++i) CHECK(seen[i] == 1, "[%s] output %d covered %d times\n", name, i, seen[i]);
+  std::printf("[%s] lds bank-conflict ways: write %d, A read %d, B read %d\n", name, cw.worst, cr_a.worst, cr_b.worst);
   CHECK(cr_a.worst == 1 && cr_b.worst == 1, "[%s] fragment reads conflict\n", name);
-  CHECK(cw_a.worst == 1 && cw_b.worst == 1, "[%s] stage writes conflict\n", name);
 }
 
 // DMA staging + ds_read_b64_tr_b16 operand path of the 16-bit kernels.
@@ -526,9 +464,9 @@ int main() {
   run_dma8();
   run_wide(2);
   run_wide(1);
-  run(2, "f16/bf16");
-  run(1, "fp8");
-  run(4, "f32");
+  run_f32(64, 256);
+  run_f32(64, 512);
+  run_f32(128, 512);
   // The direct-to-LDS load plan keeps only block 0's offsets per lane and
   // steps to block b from there: A rows +8 per block with the chunk
   // recomputed as (lane % 8) ^ ((4b + lane / 16) % 8); B rows +4 (16-bit) or

@@ -218,23 +218,12 @@ __device__ inline u32x3 split_pair(uint32_t xb, uint32_t yb) {
   return u32x3{w0, w1, __builtin_bit_cast(uint32_t, p2)};
 }
 
-// Byte offset of column n of k-row k in a plane of B: K-major like the 16-bit
-// tiles' (btr_offset); 64-column tiles keep 128 bytes per k-row and swap its
-// halves by (k / 2) % 2, so that the four k-rows of a transpose read fall in
-// distinct banks.
-template <int TM> __device__ inline int f32_b_offset(int k, int n) {
-  if constexpr (TM == 128) return btr_offset(k, n);
-  return f32_btr64_offset(k, n);
-}
-
 // One k-tile (32 k) of A and B in flight in registers: a thread holds E
 // consecutive k of one row of A and E consecutive columns of one k-row of B.
 // Every load is issued unconditionally (past M, N or K: an offset that reads
 // zero), so the compiler's count of outstanding loads stays exact.
 template <int TM, int NT> struct F32Regs {
   static constexpr int E = TM * 32 / NT;  // 8 or 4
-  static constexpr int TPA = 32 / E;      // threads per row of A
-  static constexpr int TPB = TM / E;      // threads per k-row of B
   static constexpr int V = E / 4;
   u32x4 a[V], b[V];
 
@@ -251,9 +240,9 @@ template <int TM, int NT> struct F32Regs {
     w.rb = make_rsrc(pb, b_bytes);
     w.K = K;
     w.ldb = ldb;
-    w.ak = (t % TPA) * E;
-    w.bk = t / TPB;
-    const uint32_t row = row0 + (uint32_t)(t / TPA), n = n0 + (uint32_t)((t % TPB) * E);
+    w.ak = f32_a_k(t, E);
+    w.bk = f32_b_k(t, E, TM);
+    const uint32_t row = row0 + (uint32_t)f32_a_row(t, E), n = n0 + (uint32_t)f32_b_n(t, E, TM);
     // rows past M start at or past the end of the batch slice: they read zero
     w.a_off = row < M ? row * lda + (uint32_t)w.ak * 4u : kOutOfRange;
     w.b_off = n < N ? (uint32_t)w.bk * ldb + n * 4u : kOutOfRange;
@@ -285,9 +274,8 @@ template <int TM, int NT> struct F32Regs {
   }
   // Splits the values and writes their parts to the planes of a stage.
   __device__ inline void store(uint8_t* stage, int t, Tiny& tiny) const {
-    const int row = t / TPA, ak = (t % TPA) * E, bk = t / TPB, bn = (t % TPB) * E;
-    put(a, stage + a64_lds_offset(row, ak >> 3) + (ak & 7) * 2, Cfg<DT_F32, TM>::kAPlane, tiny);
-    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_offset<TM>(bk, bn), Cfg<DT_F32, TM>::kBPlane, tiny);
+    put(a, stage + f32_a_store(t, E), Cfg<DT_F32, TM>::kAPlane, tiny);
+    put(b, stage + 3 * Cfg<DT_F32, TM>::kAPlane + f32_b_store(t, E, TM), Cfg<DT_F32, TM>::kBPlane, tiny);
   }
   static __device__ inline void put(const u32x4 (&v)[V], uint8_t* dst, int plane, Tiny& tiny) {
     u32x3 w[2 * V];
@@ -331,8 +319,8 @@ template <int TM, int MT, int NTN, int KS> struct F32Frags {
 #pragma unroll
         for (int nt = 0; nt < NTN; ++nt) {
           const uint8_t* sb = stage + 3 * AP + p * BP;
-          const u32x2 lo = tr_read(sb + f32_b_offset<TM>(btr_k(s, 0, lane), btr_n(nw + nt * 32, lane)));
-          const u32x2 hi = tr_read(sb + f32_b_offset<TM>(btr_k(s, 1, lane), btr_n(nw + nt * 32, lane)));
+          const u32x2 lo = tr_read(sb + f32_b_offset(TM, btr_k(s, 0, lane), btr_n(nw + nt * 32, lane)));
+          const u32x2 hi = tr_read(sb + f32_b_offset(TM, btr_k(s, 1, lane), btr_n(nw + nt * 32, lane)));
           b[i][p][nt] = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
       }
