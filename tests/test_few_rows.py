@@ -34,17 +34,6 @@ def test_rule(native_lib):
         assert abs(est(*inside) - est(100, inside[1])) > 0.08 * est(*inside), inside
 
 
-def test_chunks_of_a_row_fit_a_lane():
-    """A lane holds at most 7 chunks of 8 columns of a row (NC of the kernel),
-    over every shape the rule lets in."""
-    worst = 0
-    for m in range(1, 33):
-        tiles = (16384 // m - 4) // 128
-        waves = 8 if m == 1 else (4 if m == 2 else (2 if m <= 4 else 1))
-        worst = max(worst, -(-(tiles * 16) // (64 * waves)))
-    assert worst == 7
-
-
 SHAPES = [
     # one row over one tile and less, K from nothing to 128 (one and two units a tile)
     (1, 1, 8, 8), (3, 1, 128, 64), (2, 1, 136, 72), (2, 1, 264, 128), (2, 2, 200, 0),

@@ -53,7 +53,20 @@ template <int S> struct Lds {
 static_assert(Lds<6>::BYTES <= 160 * 1024 && 2 * Lds<4>::BYTES <= 160 * 1024, "LDS");
 
 // Waves that share a row in the last phase: 8 over the rows' next power of two.
-__device__ inline int waves_per_row(int m) { return m == 1 ? 8 : (m == 2 ? 4 : (m <= 4 ? 2 : 1)); }
+__host__ __device__ constexpr int waves_per_row(int m) { return m == 1 ? 8 : (m == 2 ? 4 : (m <= 4 ? 2 : 1)); }
+// The most chunks a lane holds, over every number of rows with the longest rows
+// that the logits' limit lets in: the last phase reads, sums and stores NC.
+constexpr int most_chunks() {
+  int most = 0;
+  for (int m = 1; m <= kFewRowsMax; ++m) {
+    const int tiles = (kFewRowsMaxLogits / m - kFewRowsPad) / BN, lanes = 64 * waves_per_row(m);
+    const int chunks = (tiles * (BN / 8) + lanes - 1) / lanes;
+    most = chunks > most ? chunks : most;
+  }
+  return most;
+}
+static_assert(most_chunks() == NC && kFewRowsMax <= 32, "chunks of a row in a lane's registers; 32 rows per MFMA");
+static_assert(kFewRowsPairLogits <= kFewRowsMaxLogits, "the pair limit is the smaller one");
 }  // namespace few
 
 template <int IN_DT, int OUT_DT, int S>

@@ -51,7 +51,8 @@ int exchange_lds_pad(int in_dt, int out_dt, const TileShape& ts, int64_t grid, i
 static_assert(kExchangeMaxTiles == kMaxExchangeTiles, "exchange slot limit");
 static_assert(tall_slots(DT_F32) == 2 * tall_entries(DT_F32) && tall_slots(DT_F16) == 2 * tall_entries(DT_F16),
               "slots of a 256-row tile");
-static_assert(kFewRowsLogits == kFewRowsMaxLogits && kFewRowsLogitsPair == kFewRowsPairLogits && kFewRowsPad == 4,
+static_assert(kFewRows == kFewRowsMax && kFewRowsLogits == kFewRowsMaxLogits &&
+                  kFewRowsLogitsPair == kFewRowsPairLogits && kFewRowsPad == 4,
               "few-row kernel limits");
 }  // namespace wtc
 

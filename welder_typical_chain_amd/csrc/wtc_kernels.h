@@ -66,6 +66,7 @@ int rows_kernel_max_k();
 
 // One workgroup per batch of few rows (tile_shape's rule: rows, logits that fit
 // LDS); `stages`: 6, or 4 for two workgroups per CU.
+constexpr int kFewRowsMax = 32;           // rows of a batch
 constexpr int kFewRowsMaxLogits = 16384;  // floats of logits a workgroup keeps
 constexpr int kFewRowsPairLogits = 4096;  // ... with two workgroups per CU
 constexpr int kFewRowsPad = 4;            // floats after each row: rows start in different banks
