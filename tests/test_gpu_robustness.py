@@ -214,7 +214,7 @@ def test_graph_with_default_workspace_survives_its_growth(native_lib):
     from welder_typical_chain_amd.chain import matmul_softmax
     _announce("graph on the default workspace, then the workspace grows, then replays")
     a, b = _inputs(512, 1024, 128, 7)
-    big_a, big_b = _inputs(2048, 8192, 128, 8)
+    big_a, big_b = _inputs(2048, 16384, 128, 8)
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
     out = torch.empty((512, 1024), dtype=torch.float16, device="cuda")
