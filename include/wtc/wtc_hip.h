@@ -95,7 +95,13 @@ int wtc_matmul_softmax(const void *a, const void *b, void *out, int64_t batch,
 /* Tile parameters of one kernel variant, in the fields and units of the
  * reference's best.json (compiler/scheduler/Search.cpp:62-86): a tile_m x
  * tile_n output tile per workgroup, tile_k elements of K per pipeline stage,
- * thread_tile_m x thread_tile_n accumulators per lane. */
+ * thread_tile_m x thread_tile_n accumulators per lane.  They name a variant;
+ * where a path has a form for a range of sizes, a request of that variant runs
+ * that form, and plans still report the variant's own tiles (the grid is that of
+ * the form): f32 inputs on the EXCHANGE path run 64 x 64 tiles while two per CU
+ * hold them all, the variant with loader waves runs 256 x 128 tiles on the
+ * EXCHANGE path where 128-row tiles outnumber the CUs and those do not, and the
+ * ROWS variant one workgroup per batch for at most 32 rows. */
 typedef struct wtc_tiles {
   int64_t tile_m, tile_n, tile_k, thread_tile_m, thread_tile_n;
 } wtc_tiles;

@@ -20,10 +20,10 @@
 // waves sharing the row.
 //
 // Epilogues (template parameter EPI):
-//   kEpiExchange  single pass.  Every tile publishes its per-row (max, sumexp)
-//                 to HBM, the tiles of one row block (all co-resident, the
-//                 launcher checks occupancy) meet at a counter, each merges the
-//                 row statistics and writes normalised outputs once.
+//   kEpiExchange  single pass.  The tiles of one row block (all co-resident, the
+//                 launcher checks occupancy) publish their per-row statistics as
+//                 tagged entries in HBM (exchange_entries.h), each polls and
+//                 merges the others' and writes normalised outputs once.
 //   kEpiSplit     first pass of the two-pass online softmax for rows wider
 //                 than what can be co-resident: stores exp2(y - tile_max) and
 //                 the per-tile (max, sumexp); `rescale_rows_kernel` merges the
@@ -1187,7 +1187,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
   // running max and sum as below.  kTallMaxColTiles (variants.h) keeps a row to
   // one group of U tiles per thread, whose loads are in flight together; a second
   // one is a second round trip between XCDs.  bf16 1500 x 3000 x 1000 (24 tiles a
-  // row): this kernel 24.5 us, the split path's two 20.5 and 7.5.
+  // row): this kernel 25.0 us, the split path's two 20.5 and 7.5.
   // ENT = 2 (f32 outputs): a log-sum-exp in one f32 carries the error of the
   // logarithm and of its own rounding into every output of the row (f16 1500 x
   // 3000 x 64, relative 2-norm error of the outputs 2.1e-7; split path 1.5e-7),

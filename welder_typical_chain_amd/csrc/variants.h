@@ -23,7 +23,7 @@
 namespace wtc {
 
 enum VariantId : int {
-  kVarTile128 = 0,        // 128x128 tile; 16-bit/fp8: 8 waves of 64x32, f32: 4 waves of 64x64
+  kVarTile128 = 0,        // 128x128 tile; 16-bit/fp8: 8 waves of 64x32, f32: 4 waves of 64x64 per k-group of two
   kVarTile128Loaders = 1,  // 128x128 tile, 4 MFMA waves of 64x64 + 4 loader waves (16-bit/fp8)
   kVarTile256 = 2,        // 256x128 tile, 8 waves of 64x64 (16-bit/fp8)
   kVarRows = 3,           // one 128-row block over all of n, two passes (16-bit, k <= 128)
@@ -31,7 +31,9 @@ enum VariantId : int {
   kNumVariants = 5,
 };
 
-// One variant in the reference's tile vocabulary (best.json): tile_k counts
+// One variant in the reference's tile vocabulary (best.json): what a caller asks
+// for and a plan reports.  On some paths a request runs with another tile than the
+// variant's own, by the problem's size: tile_shape (below).  tile_k counts
 // elements of the input type in one pipeline stage of K, the thread tile is
 // the accumulator footprint of one lane (rows x columns).
 struct VariantDesc {
@@ -83,7 +85,7 @@ constexpr int64_t kF32OneGroupK = 192;
 // CUs and 256-row tiles (the loader-wave variant's request, run without loader
 // waves) do not.  They may leave CUs idle, as they do on the split path, but need
 // no second pass over the output (us, split and exchange: 1500 x 3000 x 1000 bf16
-// 27.7, 24.5; 3328 x 2048 x 512 f16 25.2, 17.4; 15 x 130 x 2048 x 256 bf16 -> f32
+// 27.7, 25.3; 3328 x 2048 x 512 f16 25.2, 17.4; 15 x 130 x 2048 x 256 bf16 -> f32
 // 24.1, 16.1; 2304 x 2048 x 1024 fp8 23.9, 18.5; a tile on every CU: 4096 x 2048 x
 // 128 f16 22.3, 14.2, x 1024 32.0, 28.6, 8 x 1024 x 1024 x 512 31.5, 18.8, 4096 x
 // 2048 x 4096 fp8 46.9, 43.8; of 30 such calls timed none was slower).  Rows of

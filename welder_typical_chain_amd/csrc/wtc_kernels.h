@@ -27,7 +27,7 @@ struct ChainParams {
   int nRB;          // row blocks (of the tile's rows) per batch
   int nT;           // column tiles (of the tile's columns) per row block
   float2* partial;  // split path: [batch][nRB * tile rows][nT] per-tile row (max, sumexp), log2
-  uint64_t* ent;    // exchange path: [slot][128] tagged per-row log-sum-exp entries
+  uint64_t* ent;    // exchange path: [slot][128] tagged per-row log-sum-exp (or max, sum) entries
   uint32_t* gen;    // exchange path: [kMaxExchangeTiles] slot generation words
   uint32_t* err;    // [0] bit 0: an exchange wait timed out; [1] longest wait
                     // (100 MHz ticks); [2] number of timed-out waits
@@ -35,8 +35,8 @@ struct ChainParams {
   uint64_t spin_ticks;  // exchange wait limit, 100 MHz ticks
 };
 
-// 16-bit and fp8 inputs: 128-column tiles; tile_rows: 128, or 256 (split
-// epilogue, and f32 logits); loaders: 1 for the 128-row layout with 4 MFMA and
+// 16-bit and fp8 inputs: 128-column tiles; tile_rows: 128, or 256 (exchange and
+// split epilogues, and f32 logits); loaders: 1 for the 128-row layout with 4 MFMA and
 // 4 loader waves (exchange and split epilogues, and f32 logits).  f32 inputs:
 // tile_rows 128 (128 x 128, loaders = 1: two k-groups) or, exchange epilogue,
 // 64 (64 x 64, one or two k-groups).  NULL for a combination not built.
