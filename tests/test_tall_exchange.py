@@ -83,6 +83,14 @@ def test_slots_of_f32_outputs(native_lib):
         pl = _lib.plan(1, m, 2048, 256, _lib.DTYPE_F16, _lib.DTYPE_F32, _lib.PATH_EXCHANGE)
         assert pl["grid"] == -(-m // 256) * 16 and 4 * pl["grid"] <= 1024
         assert pl["workspace_bytes"] >= 256 + 4096 + 4 * pl["grid"] * 1024
+        size = _lib.lib().wtc_matmul_softmax_workspace_size
+        for path in (_lib.PATH_AUTO, _lib.PATH_EXCHANGE):
+            assert size(1, m, 2048, 256, _lib.DTYPE_F16, _lib.DTYPE_F32, path) >= pl["workspace_bytes"]
+    # other paths and smaller tiles ask for no more than with 16-bit outputs
+    for path, m in ((_lib.PATH_SPLIT, 2049), (_lib.PATH_EXCHANGE, 2048), (_lib.PATH_ROWS, 2049)):
+        wide, half = (_lib.plan(1, m, 2048, 64, _lib.DTYPE_F16, out, path)["workspace_bytes"]
+                      for out in (_lib.DTYPE_F32, _lib.DTYPE_F16))
+        assert wide == half
 
 
 @pytest.mark.gpu

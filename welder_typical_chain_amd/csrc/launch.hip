@@ -115,7 +115,9 @@ struct WsLayout {
   int64_t total;
 };
 
-WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int out_dt, int path) {
+// `ts`: the tile of a plan, if there is one (without: what any tile of the path needs).
+WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int out_dt, int path,
+                   const TileShape* ts = nullptr) {
   WsLayout w{};
   const int64_t nT = ceil_div(n, kTile);
   w.gen_off = kGenOff;
@@ -127,7 +129,8 @@ WsLayout ws_layout(int64_t batch, int64_t m, int64_t n, int in_dt, int out_dt, i
     const int64_t tiles = batch * ceil_div(m, 64) * ceil_div(n, 64);
     if (tiles <= kMaxExchangeTiles && tiles * kTile * 8 > exch_bytes) exch_bytes = tiles * kTile * 8;
   }
-  if (in_dt != DT_F32) {  // 256 x 128 tiles, when the exchange path runs them
+  const bool exchange = path == WTC_PATH_EXCHANGE || (!ts && path == WTC_PATH_AUTO);
+  if (in_dt != DT_F32 && exchange && (!ts || ts->rows == 256)) {  // 256 x 128 tiles
     const int64_t slots = batch * ceil_div(m, 256) * nT * tall_slots(out_dt);
     if (slots <= kMaxExchangeTiles && slots * kTile * 8 > exch_bytes) exch_bytes = slots * kTile * 8;
   }
@@ -217,7 +220,7 @@ int plan_impl(int64_t batch, int64_t m, int64_t n, int64_t k, int in_dt, int out
   out->path = c.path;
   out->ts = tile_shape(c.v, c.path, pr);
   out->grid = grid;
-  out->ws = ws_layout(batch, m, n, in_dt, out_dt, c.path).total;
+  out->ws = ws_layout(batch, m, n, in_dt, out_dt, c.path, &out->ts).total;
   out->est_us = c.est_us;
   return WTC_OK;
 }
@@ -928,7 +931,7 @@ int matmul_softmax_impl(const void* a, const void* b, void* out, int64_t batch, 
     rc = default_workspace(ds, need, &ws, stream);
     if (rc) return rc;
   }
-  const WsLayout L = ws_layout(batch, m, n, in_dtype, out_dtype, chosen);
+  const WsLayout L = ws_layout(batch, m, n, in_dtype, out_dtype, chosen, &pl.ts);
   uint8_t* wsb = static_cast<uint8_t*>(ws);
 
   const int isz = dtype_bytes(in_dtype), osz = dtype_bytes(out_dtype);
