@@ -1248,7 +1248,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
         nm = fmaxf(nm, l[u]);
       }
       const float ref = nm == -INFINITY ? 0.0f : nm;  // no entry at all in this share
-      // four partial sums: a quarter of the roundings on the way to each
+      // f32 outputs: four partial sums, a quarter of the roundings on the way to each
       float cs[4] = {*gm == -INFINITY ? 0.0f : *gs * __builtin_amdgcn_exp2f(*gm - ref), 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -1257,7 +1257,7 @@ chain_tile_kernel(const uint8_t* a_in, const uint8_t* b_in, uint32_t M32, uint32
           const int q = qb + u * P + h;
           cs[u & 3] += x * (q >= nT ? 0.0f : (q == (int)nt ? st.y : entry_value(e[1][u])));
         } else {
-          cs[u & 3] += x;
+          cs[0] += x;
         }
       }
       *gm = nm;
